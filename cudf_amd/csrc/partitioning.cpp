@@ -100,15 +100,30 @@ std::unique_ptr<mig_table> empty_like(mig_column_view const* input, int32_t num_
   return t;
 }
 
+// Bits of the partition numbers and of each counting pass over them.
+struct digit_plan {
+  int total_bits = 1;
+  int passes;
+  int bits_per_pass;
+  explicit digit_plan(uint32_t num_partitions)
+  {
+    while (total_bits < 32 && (uint64_t(1) << total_bits) < num_partitions) total_bits++;
+    passes        = (total_bits + HP_DIGIT_BITS - 1) / HP_DIGIT_BITS;
+    bits_per_pass = (total_bits + passes - 1) / passes;
+  }
+};
+
 // Regroups every column of `input` by the partition numbers in `pid` (one
 // per row, below num_partitions) with a stable LSD counting sort; writes the
-// first row of each partition to `offsets`.  The last counting pass moves up
+// first row of each partition to `offsets`.  `first_hist` holds the ranges'
+// histograms of the first digit (with room for one more counter), or is null
+// when they are yet to be counted.  The last counting pass moves up
 // to HP_MAX_MOVE_COLS fixed-width columns itself (rows read in order, values
 // written in runs per partition); validity, strings and further columns are
 // gathered afterwards through the row map.
 std::unique_ptr<mig_table> regroup(mig_column_view const* input, int32_t num_columns, int64_t n, uint32_t* pid,
-                                   uint32_t num_partitions, call_scratch& S, hipStream_t stream,
-                                   mig_memory_resource const* mr, std::vector<int32_t>& offsets)
+                                   uint32_t num_partitions, uint32_t* first_hist, call_scratch& S,
+                                   hipStream_t stream, mig_memory_resource const* mr, std::vector<int32_t>& offsets)
 {
   auto t = std::make_unique<mig_table>();
   init_table(*t, stream, mr);
@@ -152,10 +167,8 @@ std::unique_ptr<mig_table> regroup(mig_column_view const* input, int32_t num_col
     MIG_HIP_TRY(hipMemcpyAsync(d_moves, moves.data(), sizeof(hp_move_col) * moves.size(), hipMemcpyHostToDevice,
                                stream));
 
-  int total_bits = 1;
-  while (total_bits < 32 && (uint64_t(1) << total_bits) < num_partitions) total_bits++;
-  int const passes        = (total_bits + HP_DIGIT_BITS - 1) / HP_DIGIT_BITS;
-  int const bits_per_pass = (total_bits + passes - 1) / passes;
+  digit_plan const dp(num_partitions);
+  int const passes = dp.passes;
 
   uint32_t* pid_alt   = passes > 1 ? S.get<uint32_t>(n) : nullptr;
   uint32_t* rows_a    = (passes > 1 || need_map) ? S.get<uint32_t>(n) : nullptr;
@@ -169,22 +182,21 @@ std::unique_ptr<mig_table> regroup(mig_column_view const* input, int32_t num_col
   int64_t last_W            = 0;
   for (int p = 0; p < passes; p++) {
     bool const last  = p == passes - 1;
-    int const bits   = std::min(bits_per_pass, total_bits - shift);
+    int const bits   = std::min(dp.bits_per_pass, dp.total_bits - shift);
     int64_t const nd = int64_t(1) << bits;
-    // waves: enough to fill the device, few enough that the digit-major
-    // histogram stays within 2^23 counters
-    int64_t const w_cap = std::max<int64_t>(64, std::min<int64_t>(16384, (int64_t(1) << 23) / nd));
-    int64_t W           = std::min<int64_t>(w_cap, std::max<int64_t>(1, (n + 255) / 256));
-    int64_t const per   = (n + W - 1) / W;
-    W                   = (n + per - 1) / per;
-    uint32_t* hist = S.get<uint32_t>(size_t(nd * W + 1));
-    launch_hp_count(pid_cur, n, per, W, shift, bits, hist, stream);
+    hp_ranges const R = hp_plan(n, bits, num_cus_of_device());
+    int64_t const W   = R.W;
+    uint32_t* hist    = first_hist;
+    if (p > 0 || hist == nullptr) {
+      hist = S.get<uint32_t>(size_t(nd * W + 1));
+      launch_hp_count(pid_cur, n, R, shift, bits, hist, stream);
+    }
     launch_exclusive_scan_i32(reinterpret_cast<int32_t*>(hist), nd * W, reinterpret_cast<int32_t*>(hist) + nd * W,
                               stream);
     // partition numbers go out for a later pass or for the offsets of a
     // multi-pass sort (a single pass reads the offsets off its histogram);
     // the row map for a later pass or for the gathers
-    launch_hp_scatter(pid_cur, rows_cur, n, per, W, shift, bits, hist, passes == 1 ? nullptr : pid_next,
+    launch_hp_scatter(pid_cur, rows_cur, n, R, shift, bits, hist, passes == 1 ? nullptr : pid_next,
                       (!last || need_map) ? rows_next : nullptr, last ? d_moves : nullptr,
                       last ? int(moves.size()) : 0, stream);
     MIG_HIP_TRY(hipGetLastError());
@@ -275,12 +287,10 @@ void lsd_sort_rows(lsd_key const* keys, int nkeys, int64_t n, uint32_t* map, uin
     for (int p = 0; p < passes; p++) {
       int const bits   = std::min(bits_per_pass, total_bits - shift);
       int64_t const nd = int64_t(1) << bits;
-      int64_t const w_cap = std::max<int64_t>(64, std::min<int64_t>(16384, (int64_t(1) << 23) / nd));
-      int64_t W           = std::min<int64_t>(w_cap, std::max<int64_t>(1, (n + 255) / 256));
-      int64_t const per   = (n + W - 1) / W;
-      W                   = (n + per - 1) / per;
-      uint32_t* hist      = S.get<uint32_t>(size_t(nd * W + 1));
-      launch_hp_count(pid_cur, n, per, W, shift, bits, hist, s);
+      hp_ranges const R = hp_plan(n, bits, num_cus_of_device());
+      int64_t const W   = R.W;
+      uint32_t* hist    = S.get<uint32_t>(size_t(nd * W + 1));
+      launch_hp_count(pid_cur, n, R, shift, bits, hist, s);
       launch_exclusive_scan_i32(reinterpret_cast<int32_t*>(hist), nd * W, reinterpret_cast<int32_t*>(hist) + nd * W,
                                 s);
       uint32_t* rows_next = (rows_cur == rows_a) ? rows_b : rows_a;
@@ -288,7 +298,7 @@ void lsd_sort_rows(lsd_key const* keys, int nkeys, int64_t n, uint32_t* map, uin
       if (final_pass) rows_next = map;
       bool const keep_pid = p < passes - 1 || (final_pass && last_sorted);
       uint32_t* pid_out   = final_pass && last_sorted ? last_sorted : pid_next;
-      launch_hp_scatter(pid_cur, rows_cur, n, per, W, shift, bits, hist, keep_pid ? pid_out : nullptr, rows_next,
+      launch_hp_scatter(pid_cur, rows_cur, n, R, shift, bits, hist, keep_pid ? pid_out : nullptr, rows_next,
                         nullptr, 0, s);
       MIG_HIP_TRY(hipGetLastError());
       rows_cur = rows_next;
@@ -351,10 +361,13 @@ std::unique_ptr<mig_table> hash_partition(mig_column_view const* input, int32_t 
   dcol* d_cols = S.get<dcol>(h.size());
   MIG_HIP_TRY(hipMemcpyAsync(d_cols, h.data(), sizeof(dcol) * h.size(), hipMemcpyHostToDevice, stream));
   uint32_t* pid = S.get<uint32_t>(n);
-  launch_hp_partition_ids(d_cols, num_columns_to_hash, n, seed, hash_function == MIG_HASH_IDENTITY,
-                          uint32_t(num_partitions), pid, stream);
+  int const bits    = digit_plan(uint32_t(num_partitions)).bits_per_pass;
+  hp_ranges const R = hp_plan(n, bits, num_cus_of_device());
+  uint32_t* hist    = S.get<uint32_t>((size_t(R.W) << bits) + 1);
+  launch_hp_ids_count(d_cols, num_columns_to_hash, n, seed, hash_function == MIG_HASH_IDENTITY,
+                      uint32_t(num_partitions), pid, R, bits, hist, stream);
   MIG_HIP_TRY(hipGetLastError());
-  return regroup(input, num_columns, n, pid, uint32_t(num_partitions), S, stream, mr, offsets);
+  return regroup(input, num_columns, n, pid, uint32_t(num_partitions), hist, S, stream, mr, offsets);
 }
 
 std::unique_ptr<mig_table> partition_by_map(mig_column_view const* input, int32_t num_columns,
@@ -391,7 +404,7 @@ std::unique_ptr<mig_table> partition_by_map(mig_column_view const* input, int32_
   MIG_HIP_TRY(hipMemcpyAsync(&h_bad, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
   MIG_HIP_TRY(hipStreamSynchronize(stream));
   MIG_EXPECTS(h_bad == 0, "partition_map values must lie in [0, num_partitions)");
-  auto t = regroup(input, num_columns, n, pid, uint32_t(num_partitions), S, stream, mr, offsets);
+  auto t = regroup(input, num_columns, n, pid, uint32_t(num_partitions), nullptr, S, stream, mr, offsets);
   offsets.push_back(int32_t(n));
   return t;
 }

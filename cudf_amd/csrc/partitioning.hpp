@@ -17,7 +17,7 @@ struct mig_table {
 
 namespace mig {
 
-// Digit bits of one counting-sort pass (2^11 LDS counters per wave).
+// Digit bits of one counting-sort pass (2^11 16-bit LDS counters per wave).
 constexpr int HP_DIGIT_BITS = 11;
 
 // One input piece of a concatenation (device copy read by the kernels).
@@ -33,11 +33,21 @@ struct concat_piece {
   int32_t pad;
 };
 
-void launch_hp_partition_ids(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
-                             uint32_t num_partitions, uint32_t* pid, hipStream_t s);
+// How a counting pass splits its rows: W ranges of `per` rows (whole tiles of
+// rpt x 512 rows), one workgroup each.
+struct hp_ranges {
+  int rpt;
+  int64_t per;
+  int64_t W;
+};
+hp_ranges hp_plan(int64_t n, int bits, int num_cus);
+// Partition numbers of every row and the ranges' histograms of their low `bits` bits.
+void launch_hp_ids_count(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
+                         uint32_t num_partitions, uint32_t* pid, hp_ranges const& R, int bits, uint32_t* hist,
+                         hipStream_t s);
 void launch_map_partition_ids(void const* map, int32_t map_storage, int64_t n, uint32_t num_partitions,
                               uint32_t* pid, uint32_t* bad, hipStream_t s);
-void launch_hp_count(uint32_t const* pid, int64_t n, int64_t per, int64_t W, int shift, int bits, uint32_t* hist,
+void launch_hp_count(uint32_t const* pid, int64_t n, hp_ranges const& R, int shift, int bits, uint32_t* hist,
                      hipStream_t s);
 // Fixed-width column moved by the last counting pass: dst[pos] = src[row].
 struct hp_move_col {
@@ -49,8 +59,8 @@ struct hp_move_col {
 constexpr int HP_MAX_MOVE_COLS = 16;
 
 // pid_out / rows_out may be null when nothing reads them later.
-void launch_hp_scatter(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, int64_t per, int64_t W,
-                       int shift, int bits, uint32_t const* start, uint32_t* pid_out, uint32_t* rows_out,
+void launch_hp_scatter(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, hp_ranges const& R, int shift,
+                       int bits, uint32_t const* start, uint32_t* pid_out, uint32_t* rows_out,
                        hp_move_col const* move, int nmove, hipStream_t s);
 void launch_hp_offsets(uint32_t const* pid_sorted, int64_t n, uint32_t num_partitions, int32_t* offsets,
                        hipStream_t s);

@@ -3,16 +3,20 @@
 // hash_partition (cpp/src/partitioning/partitioning.cu:469-711) assigns each
 // row the partition `row_hash % num_partitions` and regroups the rows so that
 // each partition is contiguous.  Here the regrouping is a stable LSD counting
-// sort of the partition numbers, HP_DIGIT_BITS bits per pass:
-//   k_hp_count    per-wave digit histograms, written digit-major so that one
-//                 exclusive scan of the whole array gives every wave's first
-//                 output position for every digit;
-//   k_hp_scatter  every wave replays its rows in order; rows of one digit in
-//                 a 64-row chunk are ranked with ballots, so the order inside
-//                 a partition is the input row order (deterministic output).
-// One pass covers up to 2048 partitions.  Each wave owns a contiguous range
-// of rows and its own LDS counters, so no workgroup barrier orders waves.
-#include "device_ops.hpp"
+// sort of the partition numbers, HP_DIGIT_BITS bits per pass, over ranges of
+// whole tiles (one workgroup per range):
+//   k_hp_ids_count / k_hp_count  digit histogram of every range, written
+//                 digit-major so that one exclusive scan of the whole array
+//                 gives every range's first output position for every digit;
+//   k_hp_scatter  replays its range tile by tile in order; a tile's rows are
+//                 ranked stably (ballots inside a wave, per-wave counters
+//                 across waves), staged in LDS in output order and written
+//                 in runs, so the order inside a partition is the input row
+//                 order (deterministic output).
+// One pass covers up to 2048 partitions.
+#include <type_traits>
+
+#include "partition_common.hpp"
 #include "partitioning.hpp"
 
 namespace mig {
@@ -21,6 +25,9 @@ namespace {
 
 constexpr int HP_BLOCK = 256;
 constexpr int HP_WAVES = HP_BLOCK / 64;
+constexpr int HP_TILE_BLOCK = 512;  // counting and scatter kernels
+constexpr int HP_TILE_WAVES = HP_TILE_BLOCK / 64;
+constexpr int HP_MAX_RPT    = 8;    // rows per thread of a scatter tile (at most)
 
 __device__ __forceinline__ uint64_t lanes_below()
 {
@@ -56,18 +63,46 @@ __device__ __forceinline__ uint32_t identity_elem(dcol const& c, int64_t row)
   }
 }
 
-__global__ void __launch_bounds__(HP_BLOCK)
-  k_hp_partition_ids(dcol const* __restrict__ cols, int ncols, int64_t n, uint32_t seed, int identity,
-                     uint32_t num_partitions, uint32_t* __restrict__ pid)
+// Rows [r * per, min((r + 1) * per, n)) belong to range r.
+__device__ __forceinline__ void range_rows(int64_t n, int64_t per, int64_t r, int64_t& b, int64_t& e)
 {
-  int64_t const i = int64_t(blockIdx.x) * HP_BLOCK + threadIdx.x;
-  if (i >= n) return;
-  uint32_t h = seed;
-  for (int c = 0; c < ncols; c++) {
-    uint32_t const e = identity ? identity_elem(cols[c], i) : elem_hash(cols[c], i, seed);
-    h = hash_combine(h, e);
+  b = r * per;
+  e = b + per < n ? b + per : n;
+}
+
+// Digit histogram of a range from LDS, digit-major.
+__device__ __forceinline__ void store_hist(uint32_t const* cnt, uint32_t nd, int64_t W, uint32_t* hist)
+{
+  for (uint32_t d = threadIdx.x; d < nd; d += HP_TILE_BLOCK) gp(hist)[int64_t(d) * W + blockIdx.x] = cnt[d];
+}
+
+// Partition numbers of a range's rows and the histogram of their first digit
+// (one pass over the hashed columns; a separate counting pass read the
+// numbers back, 82 us at 50M rows).
+__global__ void __launch_bounds__(HP_TILE_BLOCK)
+  k_hp_ids_count(dcol const* __restrict__ cols, int ncols, int64_t n, uint32_t seed, int identity,
+                 uint32_t num_partitions, uint32_t* __restrict__ pid, int64_t per, int64_t W, uint32_t dmask,
+                 uint32_t* __restrict__ hist)
+{
+  extern __shared__ uint32_t hp_lds[];
+  uint32_t const nd = dmask + 1;
+  for (uint32_t d = threadIdx.x; d < nd; d += HP_TILE_BLOCK) hp_lds[d] = 0;
+  lds_barrier();
+  int64_t b, e;
+  range_rows(n, per, blockIdx.x, b, e);
+  bool const pow2 = (num_partitions & (num_partitions - 1)) == 0;
+  for (int64_t i = b + threadIdx.x; i < e; i += HP_TILE_BLOCK) {
+    uint32_t h = seed;
+    for (int c = 0; c < ncols; c++) {
+      uint32_t const x = identity ? identity_elem(cols[c], i) : elem_hash(cols[c], i, seed);
+      h = hash_combine(h, x);
+    }
+    uint32_t const p = pow2 ? (h & (num_partitions - 1)) : h % num_partitions;
+    gp(pid)[i]       = p;
+    __hip_atomic_fetch_add(&hp_lds[p & dmask], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  gp(pid)[i] = (num_partitions & (num_partitions - 1)) == 0 ? (h & (num_partitions - 1)) : h % num_partitions;
+  lds_barrier();
+  store_hist(hp_lds, nd, W, hist);
 }
 
 __global__ void __launch_bounds__(HP_BLOCK)
@@ -96,88 +131,187 @@ __global__ void __launch_bounds__(HP_BLOCK)
   gp(pid)[i] = ok ? uint32_t(v) : 0u;
 }
 
-// Rows [w * per, min((w + 1) * per, n)) belong to wave w.
-__device__ __forceinline__ void wave_range(int64_t n, int64_t per, int64_t w, int64_t& b, int64_t& e)
-{
-  b = w * per;
-  e = b + per < n ? b + per : n;
-  if (b > n) b = n;
-}
-
-__global__ void __launch_bounds__(HP_BLOCK)
+__global__ void __launch_bounds__(HP_TILE_BLOCK)
   k_hp_count(uint32_t const* __restrict__ pid, int64_t n, int64_t per, int64_t W, int shift, uint32_t dmask,
              uint32_t* __restrict__ hist)
 {
   extern __shared__ uint32_t hp_lds[];
-  int const wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   uint32_t const nd = dmask + 1;
-  uint32_t* cnt     = hp_lds + wave * nd;
-  for (uint32_t d = lane; d < nd; d += 64) cnt[d] = 0;
-  __syncthreads();
-  int64_t const w = int64_t(blockIdx.x) * HP_WAVES + wave;
-  int64_t b = n, e = n;
-  if (w < W) wave_range(n, per, w, b, e);
-  for (int64_t i = b + lane; i < e; i += 64) atomicAdd(&cnt[(gp(pid)[i] >> shift) & dmask], 1u);
-  __syncthreads();
-  if (w < W)
-    for (uint32_t d = lane; d < nd; d += 64) gp(hist)[int64_t(d) * W + w] = cnt[d];
+  for (uint32_t d = threadIdx.x; d < nd; d += HP_TILE_BLOCK) hp_lds[d] = 0;
+  lds_barrier();
+  int64_t b, e;
+  range_rows(n, per, blockIdx.x, b, e);
+  for (int64_t i = b + threadIdx.x; i < e; i += HP_TILE_BLOCK)
+    __hip_atomic_fetch_add(&hp_lds[(gp(pid)[i] >> shift) & dmask], 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+  lds_barrier();
+  store_hist(hp_lds, nd, W, hist);
 }
 
-__global__ void __launch_bounds__(HP_BLOCK)
+// One value stream of a tile: loaded in input order (row of each of the
+// thread's elements in `row`), staged at the elements' output-order positions
+// `lp` and written so that consecutive threads store consecutive elements of
+// a run (`dst` is the output index of position k * block + thread).
+template <typename T, int RPT, typename F>
+__device__ __forceinline__ void move_tile(uint8_t* stage_bytes, uint32_t live, uint16_t const (&lp)[RPT],
+                                          uint32_t const (&dst)[RPT], int total, gmem<T>* out, int64_t stride,
+                                          int64_t off, F&& load)
+{
+  T* const stage = reinterpret_cast<T*>(stage_bytes);
+  T v[RPT];
+#pragma unroll
+  for (int k = 0; k < RPT; k++)
+    if ((live >> k) & 1u) v[k] = load(k);
+#pragma unroll
+  for (int k = 0; k < RPT; k++)
+    if ((live >> k) & 1u) stage[lp[k]] = v[k];
+  lds_barrier();
+#pragma unroll
+  for (int k = 0; k < RPT; k++) {
+    int const j = k * HP_TILE_BLOCK + int(threadIdx.x);
+    if (j < total) out[int64_t(dst[k]) * stride + off] = stage[j];
+  }
+  lds_barrier();
+}
+
+// One counting pass over a range.  Bound by memory: every value is read and
+// written once, and without staging each lane stored its element to a line
+// of its own (64 / partitions elements per run), which at 256 partitions and
+// 20-byte rows moved 50M rows in 2.9 ms.  A tile of RPT x 512 rows staged in
+// LDS gives runs of RPT * 512 / partitions rows, and since a workgroup owns a
+// contiguous range, consecutive tiles continue its runs (the partial lines at
+// a run's ends meet in the same L2).  56 KB of LDS at 2048 digits, 42 KB at
+// 256: two to three workgroups per CU.
+template <int RPT>
+__global__ void __launch_bounds__(HP_TILE_BLOCK)
   k_hp_scatter(uint32_t const* __restrict__ pid_in, uint32_t const* __restrict__ rows_in, int64_t n, int64_t per,
                int64_t W, int shift, int bits, uint32_t const* __restrict__ start, uint32_t* __restrict__ pid_out,
                uint32_t* __restrict__ rows_out, hp_move_col const* __restrict__ move, int nmove)
 {
-  extern __shared__ uint32_t hp_lds[];
-  int const wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int T = RPT * HP_TILE_BLOCK;
+  extern __shared__ __attribute__((aligned(16))) uint8_t hp_tile_lds[];
+  __shared__ uint32_t wave_sum[HP_TILE_WAVES];
   uint32_t const dmask = (1u << bits) - 1u;
-  uint32_t const nd    = dmask + 1;
-  volatile uint32_t* next = hp_lds + wave * nd;
-  int64_t const w = int64_t(blockIdx.x) * HP_WAVES + wave;
-  if (w >= W) return;
-  for (uint32_t d = lane; d < nd; d += 64) next[d] = gp(start)[int64_t(d) * W + w];
-  __builtin_amdgcn_wave_barrier();
+  int const nd         = int(dmask) + 1;
+  // the per-wave counters are dead once every row has its position; the
+  // value stage takes their place
+  int const stage_bytes = T * 8 > HP_TILE_WAVES * nd * 2 ? T * 8 : HP_TILE_WAVES * nd * 2;
+  uint8_t* const stage  = hp_tile_lds;
+  auto* const next      = reinterpret_cast<uint32_t*>(hp_tile_lds + stage_bytes);  // next output index per digit
+  auto* const delta     = next + nd;  // output index minus position, of a digit's rows in this tile
+  auto* const sdig      = reinterpret_cast<uint16_t*>(delta + nd);
+  int const tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  volatile uint16_t* const wcnt = reinterpret_cast<uint16_t*>(hp_tile_lds) + wave * nd;
+  auto* const cnt16             = reinterpret_cast<uint16_t*>(hp_tile_lds);
+  for (int d = tid; d < nd; d += HP_TILE_BLOCK) next[d] = gp(start)[int64_t(d) * W + blockIdx.x];
   int64_t b, e;
-  wave_range(n, per, w, b, e);
+  range_rows(n, per, blockIdx.x, b, e);
   uint64_t const below = lanes_below();
-  for (int64_t i0 = b; i0 < e; i0 += 64) {
-    int64_t const i  = i0 + lane;
-    bool const valid = i < e;
-    uint32_t const p   = valid ? gp(pid_in)[i] : 0u;
-    uint32_t const row = valid ? (rows_in ? gp(rows_in)[i] : uint32_t(i)) : 0u;
-    uint32_t const d   = (p >> shift) & dmask;
-    // lanes holding the same digit
-    uint64_t peers = __ballot(valid);
-    for (int k = 0; k < bits; k++) {
-      uint64_t const set = __ballot(valid && ((d >> k) & 1u));
-      peers &= ((d >> k) & 1u) ? set : ~set;
-    }
-    uint32_t base = 0;
-    if (valid) base = next[d];
-    __builtin_amdgcn_wave_barrier();
-    if (valid) {
-      uint32_t const pos = base + uint32_t(__popcll(peers & below));
-      if (pid_out) gp(pid_out)[pos] = p;  // needed by a later pass or the offsets kernel only
-      if (rows_out) gp(rows_out)[pos] = row;
-      // the last pass moves fixed-width values straight to their place
-      for (int c = 0; c < nmove; c++) {
-        hp_move_col const mc = move[c];
-        switch (mc.width) {
-          case 1: gp(static_cast<uint8_t*>(mc.dst))[pos] = gp(static_cast<uint8_t const*>(mc.src))[row]; break;
-          case 2: gp(static_cast<uint16_t*>(mc.dst))[pos] = gp(static_cast<uint16_t const*>(mc.src))[row]; break;
-          case 4: gp(static_cast<uint32_t*>(mc.dst))[pos] = gp(static_cast<uint32_t const*>(mc.src))[row]; break;
-          case 8: gp(static_cast<uint64_t*>(mc.dst))[pos] = gp(static_cast<uint64_t const*>(mc.src))[row]; break;
-          default: {
-            uint64_t const lo = gp(static_cast<uint64_t const*>(mc.src))[2 * int64_t(row)];
-            uint64_t const hi = gp(static_cast<uint64_t const*>(mc.src))[2 * int64_t(row) + 1];
-            gp(static_cast<uint64_t*>(mc.dst))[2 * int64_t(pos)]     = lo;
-            gp(static_cast<uint64_t*>(mc.dst))[2 * int64_t(pos) + 1] = hi;
-          }
-        }
+  int const per_t      = (nd + HP_TILE_BLOCK - 1) / HP_TILE_BLOCK;  // digits per thread of the scan
+  for (int64_t t0 = b; t0 < e; t0 += T) {
+    int const total = e - t0 < T ? int(e - t0) : T;
+    for (int d = lane; d < nd; d += 64) wcnt[d] = 0;
+    // wave w takes the rows [w * 64 * RPT, (w + 1) * 64 * RPT) of the tile
+    uint32_t p[RPT], row[RPT];
+    uint16_t lp[RPT];
+    uint32_t live = 0;
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+      int const j = (wave * RPT + k) * 64 + lane;
+      p[k]        = 0;
+      row[k]      = 0;
+      if (j < total) {
+        live |= 1u << k;
+        p[k]   = gp(pid_in)[t0 + j];
+        row[k] = rows_in ? gp(rows_in)[t0 + j] : uint32_t(t0 + j);
       }
-      if ((peers & below) == 0) next[d] = base + uint32_t(__popcll(peers));
     }
     __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {  // stable rank among the wave's rows of the digit
+      bool const valid = (live >> k) & 1u;
+      uint32_t const d = (p[k] >> shift) & dmask;
+      uint64_t peers   = __ballot(valid);
+      for (int q = 0; q < bits; q++) {
+        uint64_t const set = __ballot(valid && ((d >> q) & 1u));
+        peers &= ((d >> q) & 1u) ? set : ~set;
+      }
+      uint32_t first = 0;
+      if (valid) first = wcnt[d];
+      __builtin_amdgcn_wave_barrier();
+      lp[k] = uint16_t(first + uint32_t(__popcll(peers & below)));
+      if (valid && (peers & below) == 0) wcnt[d] = uint16_t(first + uint32_t(__popcll(peers)));
+      __builtin_amdgcn_wave_barrier();
+    }
+    lds_barrier();
+    // rows per digit over the waves, then each wave's first position per digit
+    uint32_t sum = 0;
+    for (int q = 0; q < per_t; q++) {
+      int const d = tid * per_t + q;
+      if (d < nd)
+        for (int w = 0; w < HP_TILE_WAVES; w++) sum += cnt16[w * nd + d];
+    }
+    uint32_t incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      uint32_t const y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wave_sum[wave] = incl;
+    lds_barrier();
+    uint32_t run = incl - sum;
+    for (int w = 0; w < wave; w++) run += wave_sum[w];
+    for (int q = 0; q < per_t; q++) {
+      int const d = tid * per_t + q;
+      if (d >= nd) break;
+      uint32_t const first = run;
+      for (int w = 0; w < HP_TILE_WAVES; w++) {
+        uint32_t const c  = cnt16[w * nd + d];
+        cnt16[w * nd + d] = uint16_t(run);
+        run += c;
+      }
+      delta[d] = next[d] - first;
+      next[d] += run - first;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+      if (!((live >> k) & 1u)) continue;
+      uint32_t const d = (p[k] >> shift) & dmask;
+      lp[k]            = uint16_t(lp[k] + wcnt[d]);
+      sdig[lp[k]]      = uint16_t(d);
+    }
+    lds_barrier();  // the counters become the stage
+    uint32_t dst[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+      int const j = k * HP_TILE_BLOCK + tid;
+      dst[k]      = j < total ? delta[sdig[j]] + uint32_t(j) : 0u;
+    }
+    if (pid_out)  // needed by a later pass or the offsets kernel only
+      move_tile<uint32_t, RPT>(stage, live, lp, dst, total, gp(pid_out), 1, 0, [&](int k) { return p[k]; });
+    if (rows_out)
+      move_tile<uint32_t, RPT>(stage, live, lp, dst, total, gp(rows_out), 1, 0, [&](int k) { return row[k]; });
+    // the last pass moves fixed-width values straight to their place
+    for (int c = 0; c < nmove; c++) {
+      hp_move_col const mc = move[c];
+      auto from = [&](auto* typed) {
+        using V = std::remove_const_t<std::remove_pointer_t<decltype(typed)>>;
+        move_tile<V, RPT>(stage, live, lp, dst, total, gp(static_cast<V*>(mc.dst)), 1, 0,
+                          [&](int k) { return gp(static_cast<V const*>(mc.src))[row[k]]; });
+      };
+      switch (mc.width) {
+        case 1: from(static_cast<uint8_t const*>(nullptr)); break;
+        case 2: from(static_cast<uint16_t const*>(nullptr)); break;
+        case 4: from(static_cast<uint32_t const*>(nullptr)); break;
+        case 8: from(static_cast<uint64_t const*>(nullptr)); break;
+        default:  // 16 bytes as two halves
+          for (int h = 0; h < 2; h++)
+            move_tile<uint64_t, RPT>(stage, live, lp, dst, total, gp(static_cast<uint64_t*>(mc.dst)), 2, h, [&](int k) {
+              return gp(static_cast<uint64_t const*>(mc.src))[2 * int64_t(row[k]) + h];
+            });
+      }
+    }
+    if (!pid_out && !rows_out && nmove == 0) lds_barrier();  // the stage's last barrier otherwise
   }
 }
 
@@ -364,12 +498,29 @@ inline unsigned mask_grid(int64_t n) { return unsigned(std::min<int64_t>(grid_of
 
 }  // namespace
 
-void launch_hp_partition_ids(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
-                             uint32_t num_partitions, uint32_t* pid, hipStream_t s)
+hp_ranges hp_plan(int64_t n, int bits, int num_cus)
+{
+  hp_ranges r;
+  // two tiles per CU at least: fewer rows take shorter tiles
+  r.rpt = HP_MAX_RPT;
+  while (r.rpt > 1 && n < int64_t(HP_TILE_BLOCK) * r.rpt * 2 * num_cus) r.rpt /= 2;
+  int64_t const tile  = int64_t(HP_TILE_BLOCK) * r.rpt;
+  int64_t const tiles = (n + tile - 1) / tile;
+  // ranges: four rounds of the three workgroups a CU holds, and a digit-major
+  // histogram of at most 2^22 counters
+  int64_t const most = std::max<int64_t>(64, std::min<int64_t>(int64_t(num_cus) * 12, (int64_t(1) << 22) >> bits));
+  r.per = (tiles + most - 1) / most * tile;
+  r.W   = (n + r.per - 1) / r.per;
+  return r;
+}
+
+void launch_hp_ids_count(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
+                         uint32_t num_partitions, uint32_t* pid, hp_ranges const& R, int bits, uint32_t* hist,
+                         hipStream_t s)
 {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_hp_partition_ids, dim3(grid_of(n)), dim3(HP_BLOCK), 0, s, d_cols, ncols, n, seed,
-                     identity ? 1 : 0, num_partitions, pid);
+  hipLaunchKernelGGL(k_hp_ids_count, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), sizeof(uint32_t) << bits, s, d_cols,
+                     ncols, n, seed, identity ? 1 : 0, num_partitions, pid, R.per, R.W, (1u << bits) - 1u, hist);
 }
 
 void launch_map_partition_ids(void const* map, int32_t map_storage, int64_t n, uint32_t num_partitions,
@@ -380,23 +531,34 @@ void launch_map_partition_ids(void const* map, int32_t map_storage, int64_t n, u
                      num_partitions, pid, bad);
 }
 
-void launch_hp_count(uint32_t const* pid, int64_t n, int64_t per, int64_t W, int shift, int bits, uint32_t* hist,
+void launch_hp_count(uint32_t const* pid, int64_t n, hp_ranges const& R, int shift, int bits, uint32_t* hist,
                      hipStream_t s)
 {
-  size_t const lds = size_t(HP_WAVES) * (size_t(1) << bits) * sizeof(uint32_t);
-  unsigned const blocks = unsigned((W + HP_WAVES - 1) / HP_WAVES);
-  hipLaunchKernelGGL(k_hp_count, dim3(blocks), dim3(HP_BLOCK), lds, s, pid, n, per, W, shift,
-                     (1u << bits) - 1u, hist);
+  hipLaunchKernelGGL(k_hp_count, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), sizeof(uint32_t) << bits, s, pid, n,
+                     R.per, R.W, shift, (1u << bits) - 1u, hist);
 }
 
-void launch_hp_scatter(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, int64_t per, int64_t W,
-                       int shift, int bits, uint32_t const* start, uint32_t* pid_out, uint32_t* rows_out,
+template <int RPT>
+static void launch_scatter_form(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, hp_ranges const& R,
+                                int shift, int bits, uint32_t const* start, uint32_t* pid_out, uint32_t* rows_out,
+                                hp_move_col const* move, int nmove, hipStream_t s)
+{
+  constexpr size_t T = size_t(RPT) * HP_TILE_BLOCK;
+  size_t const nd    = size_t(1) << bits;
+  size_t const lds   = std::max(T * 8, HP_TILE_WAVES * nd * 2) + nd * 8 + T * 2;
+  hipLaunchKernelGGL(k_hp_scatter<RPT>, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), lds, s, pid_in, rows_in, n, R.per,
+                     R.W, shift, bits, start, pid_out, rows_out, move, nmove);
+}
+
+void launch_hp_scatter(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, hp_ranges const& R, int shift,
+                       int bits, uint32_t const* start, uint32_t* pid_out, uint32_t* rows_out,
                        hp_move_col const* move, int nmove, hipStream_t s)
 {
-  size_t const lds = size_t(HP_WAVES) * (size_t(1) << bits) * sizeof(uint32_t);
-  unsigned const blocks = unsigned((W + HP_WAVES - 1) / HP_WAVES);
-  hipLaunchKernelGGL(k_hp_scatter, dim3(blocks), dim3(HP_BLOCK), lds, s, pid_in, rows_in, n, per, W, shift,
-                     bits, start, pid_out, rows_out, move, nmove);
+  auto const form = R.rpt == 8 ? launch_scatter_form<8>
+                    : R.rpt == 4 ? launch_scatter_form<4>
+                    : R.rpt == 2 ? launch_scatter_form<2>
+                                 : launch_scatter_form<1>;
+  form(pid_in, rows_in, n, R, shift, bits, start, pid_out, rows_out, move, nmove, s);
 }
 
 void launch_hp_offsets(uint32_t const* pid_sorted, int64_t n, uint32_t num_partitions, int32_t* offsets,

@@ -335,3 +335,14 @@ def test_dask_style_groupby_errors():
     k = ca.Table([ca.Column.from_numpy(np.arange(5, dtype=np.int32))])
     with pytest.raises(ValueError):
         groupby_agg([(k, {"a": ca.Column.from_numpy(np.arange(5.0))})], {"a": ["median"]})
+
+
+@pytest.mark.parametrize("nparts", [2, 255, 2048])
+@pytest.mark.parametrize("rows", [1, 511, 513, (1 << 19) - 1, (1 << 19) + 1, (1 << 20) + 513, (1 << 21) + 4097])
+def test_partition_tile_edges(rows, nparts):
+    """Scatter tiles of 512 to 4,096 rows (by input size) with partial last
+    tiles, element widths of 1 to 8 bytes: exact against the oracle."""
+    rng = np.random.default_rng(rows + nparts)
+    cols = [host_col(rng.integers(0, 1 << 40, rows)), host_col(rng.integers(-100, 100, rows).astype(np.int8)),
+            host_col(rng.integers(0, 9, rows).astype(np.int16)), host_col(rng.normal(size=rows).astype(np.float32))]
+    _check_hash_partition(cols, [0], nparts)
