@@ -364,7 +364,7 @@ std::unique_ptr<mig_table> hash_partition(mig_column_view const* input, int32_t 
   int const bits    = digit_plan(uint32_t(num_partitions)).bits_per_pass;
   hp_ranges const R = hp_plan(n, bits, num_cus_of_device());
   uint32_t* hist    = S.get<uint32_t>((size_t(R.W) << bits) + 1);
-  launch_hp_ids_count(d_cols, num_columns_to_hash, n, seed, hash_function == MIG_HASH_IDENTITY,
+  launch_hp_ids_count(d_cols, num_columns_to_hash, h[0].storage, n, seed, hash_function == MIG_HASH_IDENTITY,
                       uint32_t(num_partitions), pid, R, bits, hist, stream);
   MIG_HIP_TRY(hipGetLastError());
   return regroup(input, num_columns, n, pid, uint32_t(num_partitions), hist, S, stream, mr, offsets);

@@ -41,8 +41,9 @@ struct hp_ranges {
   int64_t W;
 };
 hp_ranges hp_plan(int64_t n, int bits, int num_cus);
-// Partition numbers of every row and the ranges' histograms of their low `bits` bits.
-void launch_hp_ids_count(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
+// Partition numbers of every row and the ranges' histograms of their low
+// `bits` bits (`storage`: the first column's).
+void launch_hp_ids_count(dcol const* d_cols, int ncols, int32_t storage, int64_t n, uint32_t seed, bool identity,
                          uint32_t num_partitions, uint32_t* pid, hp_ranges const& R, int bits, uint32_t* hist,
                          hipStream_t s);
 void launch_map_partition_ids(void const* map, int32_t map_storage, int64_t n, uint32_t num_partitions,

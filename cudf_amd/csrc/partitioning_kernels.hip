@@ -14,8 +14,6 @@
 //                 in runs, so the order inside a partition is the input row
 //                 order (deterministic output).
 // One pass covers up to 2048 partitions.
-#include <type_traits>
-
 #include "partition_common.hpp"
 #include "partitioning.hpp"
 
@@ -78,7 +76,11 @@ __device__ __forceinline__ void store_hist(uint32_t const* cnt, uint32_t nd, int
 
 // Partition numbers of a range's rows and the histogram of their first digit
 // (one pass over the hashed columns; a separate counting pass read the
-// numbers back, 82 us at 50M rows).
+// numbers back, 82 us at 50M rows).  ST is the storage of a single MurmurHash3
+// column, or ST_NONE for any columns and either hash: with the storage read
+// per row the pass is bound by its scalar and vector instructions (193 us at
+// 50M int64 rows, against 157 us with the storage fixed).
+template <int ST>
 __global__ void __launch_bounds__(HP_TILE_BLOCK)
   k_hp_ids_count(dcol const* __restrict__ cols, int ncols, int64_t n, uint32_t seed, int identity,
                  uint32_t num_partitions, uint32_t* __restrict__ pid, int64_t per, int64_t W, uint32_t dmask,
@@ -91,15 +93,36 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
   int64_t b, e;
   range_rows(n, per, blockIdx.x, b, e);
   bool const pow2 = (num_partitions & (num_partitions - 1)) == 0;
-  for (int64_t i = b + threadIdx.x; i < e; i += HP_TILE_BLOCK) {
-    uint32_t h = seed;
-    for (int c = 0; c < ncols; c++) {
-      uint32_t const x = identity ? identity_elem(cols[c], i) : elem_hash(cols[c], i, seed);
-      h = hash_combine(h, x);
+  constexpr int U = 4;  // rows in flight per thread
+  for (int64_t i0 = b + threadIdx.x; i0 < e; i0 += U * HP_TILE_BLOCK) {
+    uint32_t h[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) h[u] = seed;
+    if constexpr (ST != ST_NONE) {
+      dcol col    = cols[0];
+      col.storage = ST;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        int64_t const i = i0 + u * HP_TILE_BLOCK;
+        if (i < e) h[u] = hash_combine(seed, elem_hash(col, i, seed));
+      }
     }
-    uint32_t const p = pow2 ? (h & (num_partitions - 1)) : h % num_partitions;
-    gp(pid)[i]       = p;
-    __hip_atomic_fetch_add(&hp_lds[p & dmask], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (int c = 0; ST == ST_NONE && c < ncols; c++) {
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        int64_t const i = i0 + u * HP_TILE_BLOCK;
+        if (i >= e) continue;
+        h[u] = hash_combine(h[u], identity ? identity_elem(cols[c], i) : elem_hash(cols[c], i, seed));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      int64_t const i = i0 + u * HP_TILE_BLOCK;
+      if (i >= e) continue;
+      uint32_t const p = pow2 ? (h[u] & (num_partitions - 1)) : h[u] % num_partitions;
+      gp(pid)[i]       = p;
+      __hip_atomic_fetch_add(&hp_lds[p & dmask], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
   }
   lds_barrier();
   store_hist(hp_lds, nd, W, hist);
@@ -148,41 +171,63 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
   store_hist(hp_lds, nd, W, hist);
 }
 
-// One value stream of a tile: loaded in input order (row of each of the
-// thread's elements in `row`), staged at the elements' output-order positions
-// `lp` and written so that consecutive threads store consecutive elements of
-// a run (`dst` is the output index of position k * block + thread).
-template <typename T, int RPT, typename F>
-__device__ __forceinline__ void move_tile(uint8_t* stage_bytes, uint32_t live, uint16_t const (&lp)[RPT],
-                                          uint32_t const (&dst)[RPT], int total, gmem<T>* out, int64_t stride,
-                                          int64_t off, F&& load)
+// Values of one moved column for the thread's rows of a tile, zero-extended
+// (the low half of 16-byte elements when `half` is 0, else the high half).
+// Without a row map the tile's rows are t0 + (the thread's places), so the
+// offsets fit 32 bits and the base is uniform.
+template <int RPT, bool MAPPED>
+__device__ __forceinline__ void load_moved(hp_move_col const& mc, int half, int64_t t0, uint32_t live,
+                                           uint32_t const (&row)[RPT], uint64_t (&raw)[RPT])
 {
-  T* const stage = reinterpret_cast<T*>(stage_bytes);
-  T v[RPT];
+  auto from = [&](auto* src, int stride) {
+    auto const s = gp(src) + (MAPPED ? 0 : t0 * stride) + half;
+#pragma unroll
+    for (int k = 0; k < RPT; k++)
+      if ((live >> k) & 1u) raw[k] = MAPPED ? s[int64_t(row[k]) * stride] : s[row[k] * uint32_t(stride)];
+  };
+  switch (mc.width) {
+    case 1: from(static_cast<uint8_t const*>(mc.src), 1); break;
+    case 2: from(static_cast<uint16_t const*>(mc.src), 1); break;
+    case 4: from(static_cast<uint32_t const*>(mc.src), 1); break;
+    case 8: from(static_cast<uint64_t const*>(mc.src), 1); break;
+    default: from(static_cast<uint64_t const*>(mc.src), 2); break;
+  }
+}
+
+// The thread's elements into the stage, at their output-order positions.
+template <typename T, int RPT, typename V>
+__device__ __forceinline__ void stage_tile(uint8_t* stage, uint32_t live, uint32_t const (&lp)[RPT], V const (&v)[RPT])
+{
 #pragma unroll
   for (int k = 0; k < RPT; k++)
-    if ((live >> k) & 1u) v[k] = load(k);
-#pragma unroll
-  for (int k = 0; k < RPT; k++)
-    if ((live >> k) & 1u) stage[lp[k]] = v[k];
-  lds_barrier();
+    if ((live >> k) & 1u) reinterpret_cast<T*>(stage)[lp[k]] = T(v[k]);
+}
+
+// The staged tile to its place: consecutive threads store consecutive
+// elements of a run (`dst` is the output index of position k * block + thread).
+template <typename T, int RPT>
+__device__ __forceinline__ void store_tile(uint8_t const* stage, int tid, uint32_t const (&dst)[RPT], int total,
+                                           void* out, int64_t stride, int64_t off)
+{
+  auto const o = gp(static_cast<T*>(out)) + off;
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
-    int const j = k * HP_TILE_BLOCK + int(threadIdx.x);
-    if (j < total) out[int64_t(dst[k]) * stride + off] = stage[j];
+    int const j = k * HP_TILE_BLOCK + tid;
+    if (j < total) o[int64_t(dst[k]) * stride] = reinterpret_cast<T const*>(stage)[j];
   }
-  lds_barrier();
 }
 
 // One counting pass over a range.  Bound by memory: every value is read and
-// written once, and without staging each lane stored its element to a line
-// of its own (64 / partitions elements per run), which at 256 partitions and
-// 20-byte rows moved 50M rows in 2.9 ms.  A tile of RPT x 512 rows staged in
-// LDS gives runs of RPT * 512 / partitions rows, and since a workgroup owns a
-// contiguous range, consecutive tiles continue its runs (the partial lines at
-// a run's ends meet in the same L2).  56 KB of LDS at 2048 digits, 42 KB at
-// 256: two to three workgroups per CU.
-template <int RPT>
+// written once.  Storing each element from its own lane (runs of 64 /
+// partitions elements) moved 50M 20-byte rows into 256 partitions in 2.9 ms;
+// a tile of RPT x 512 rows staged in LDS gives runs of RPT * 512 / partitions
+// rows, and since a workgroup owns a contiguous range, consecutive tiles
+// continue its runs: 0.83 ms (2.7 TB/s), 0.44 ms into 2 partitions
+// (5 TB/s: what is left is the partial lines at the runs' ends).  Tiles of
+// 4,096 rows beat 2,048 from 64 partitions on (1.10 against 1.28 ms a call at
+// 256, 1.30 against 1.47 at 500) and tie below.  56 KB of LDS at 2048 digits,
+// 42 KB at 256, and 102 registers: two workgroups per CU.
+template <int RPT, bool MAPPED>
 __global__ void __launch_bounds__(HP_TILE_BLOCK)
   k_hp_scatter(uint32_t const* __restrict__ pid_in, uint32_t const* __restrict__ rows_in, int64_t n, int64_t per,
                int64_t W, int shift, int bits, uint32_t const* __restrict__ start, uint32_t* __restrict__ pid_out,
@@ -200,20 +245,24 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
   auto* const next      = reinterpret_cast<uint32_t*>(hp_tile_lds + stage_bytes);  // next output index per digit
   auto* const delta     = next + nd;  // output index minus position, of a digit's rows in this tile
   auto* const sdig      = reinterpret_cast<uint16_t*>(delta + nd);
-  int const tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  volatile uint16_t* const wcnt = reinterpret_cast<uint16_t*>(hp_tile_lds) + wave * nd;
+  volatile uint16_t* const wcnt = reinterpret_cast<uint16_t*>(hp_tile_lds) + (threadIdx.x >> 6) * nd;
   auto* const cnt16             = reinterpret_cast<uint16_t*>(hp_tile_lds);
-  for (int d = tid; d < nd; d += HP_TILE_BLOCK) next[d] = gp(start)[int64_t(d) * W + blockIdx.x];
+  for (int d = threadIdx.x; d < nd; d += HP_TILE_BLOCK) next[d] = gp(start)[int64_t(d) * W + blockIdx.x];
   int64_t b, e;
   range_rows(n, per, blockIdx.x, b, e);
   uint64_t const below = lanes_below();
   int const per_t      = (nd + HP_TILE_BLOCK - 1) / HP_TILE_BLOCK;  // digits per thread of the scan
   for (int64_t t0 = b; t0 < e; t0 += T) {
     int const total = e - t0 < T ? int(e - t0) : T;
+    // opaque per tile: otherwise the offsets of every row, element width and
+    // column are computed once and kept (180 registers instead of 102)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    int const wave = tid >> 6, lane = tid & 63;
     for (int d = lane; d < nd; d += 64) wcnt[d] = 0;
     // wave w takes the rows [w * 64 * RPT, (w + 1) * 64 * RPT) of the tile
-    uint32_t p[RPT], row[RPT];
-    uint16_t lp[RPT];
+    uint32_t p[RPT], row[RPT], lp[RPT];
+    uint64_t raw[RPT];
     uint32_t live = 0;
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
@@ -223,24 +272,30 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
       if (j < total) {
         live |= 1u << k;
         p[k]   = gp(pid_in)[t0 + j];
-        row[k] = rows_in ? gp(rows_in)[t0 + j] : uint32_t(t0 + j);
+        row[k] = MAPPED ? gp(rows_in)[t0 + j] : uint32_t(j);
       }
     }
+    // the first column's loads overlap the ranking
+    if (nmove > 0) load_moved<RPT, MAPPED>(move[0], 0, t0, live, row, raw);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int k = 0; k < RPT; k++) {  // stable rank among the wave's rows of the digit
       bool const valid = (live >> k) & 1u;
       uint32_t const d = (p[k] >> shift) & dmask;
       uint64_t peers   = __ballot(valid);
-      for (int q = 0; q < bits; q++) {
-        uint64_t const set = __ballot(valid && ((d >> q) & 1u));
-        peers &= ((d >> q) & 1u) ? set : ~set;
+#pragma unroll
+      for (int q = 0; q < HP_DIGIT_BITS; q++) {
+        if (q >= bits) break;
+        int32_t const bit  = int32_t(d << (31 - q)) >> 31;  // all ones when bit q is set
+        uint64_t const set = __ballot(bit != 0);
+        peers &= ~(set ^ uint64_t(int64_t(bit)));
       }
       uint32_t first = 0;
       if (valid) first = wcnt[d];
       __builtin_amdgcn_wave_barrier();
-      lp[k] = uint16_t(first + uint32_t(__popcll(peers & below)));
-      if (valid && (peers & below) == 0) wcnt[d] = uint16_t(first + uint32_t(__popcll(peers)));
+      uint32_t const ahead = uint32_t(__popcll(peers & below));
+      lp[k]                = first + ahead;
+      if (valid && ahead == 0) wcnt[d] = uint16_t(first + uint32_t(__popcll(peers)));
       __builtin_amdgcn_wave_barrier();
     }
     lds_barrier();
@@ -277,8 +332,8 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
     for (int k = 0; k < RPT; k++) {
       if (!((live >> k) & 1u)) continue;
       uint32_t const d = (p[k] >> shift) & dmask;
-      lp[k]            = uint16_t(lp[k] + wcnt[d]);
-      sdig[lp[k]]      = uint16_t(d);
+      lp[k] += wcnt[d];
+      sdig[lp[k]] = uint16_t(d);
     }
     lds_barrier();  // the counters become the stage
     uint32_t dst[RPT];
@@ -287,29 +342,48 @@ __global__ void __launch_bounds__(HP_TILE_BLOCK)
       int const j = k * HP_TILE_BLOCK + tid;
       dst[k]      = j < total ? delta[sdig[j]] + uint32_t(j) : 0u;
     }
-    if (pid_out)  // needed by a later pass or the offsets kernel only
-      move_tile<uint32_t, RPT>(stage, live, lp, dst, total, gp(pid_out), 1, 0, [&](int k) { return p[k]; });
-    if (rows_out)
-      move_tile<uint32_t, RPT>(stage, live, lp, dst, total, gp(rows_out), 1, 0, [&](int k) { return row[k]; });
-    // the last pass moves fixed-width values straight to their place
-    for (int c = 0; c < nmove; c++) {
-      hp_move_col const mc = move[c];
-      auto from = [&](auto* typed) {
-        using V = std::remove_const_t<std::remove_pointer_t<decltype(typed)>>;
-        move_tile<V, RPT>(stage, live, lp, dst, total, gp(static_cast<V*>(mc.dst)), 1, 0,
-                          [&](int k) { return gp(static_cast<V const*>(mc.src))[row[k]]; });
-      };
-      switch (mc.width) {
-        case 1: from(static_cast<uint8_t const*>(nullptr)); break;
-        case 2: from(static_cast<uint16_t const*>(nullptr)); break;
-        case 4: from(static_cast<uint32_t const*>(nullptr)); break;
-        case 8: from(static_cast<uint64_t const*>(nullptr)); break;
-        default:  // 16 bytes as two halves
-          for (int h = 0; h < 2; h++)
-            move_tile<uint64_t, RPT>(stage, live, lp, dst, total, gp(static_cast<uint64_t*>(mc.dst)), 2, h, [&](int k) {
-              return gp(static_cast<uint64_t const*>(mc.src))[2 * int64_t(row[k]) + h];
-            });
+    if (pid_out) {  // needed by a later pass or the offsets kernel only
+      stage_tile<uint32_t, RPT>(stage, live, lp, p);
+      lds_barrier();
+      store_tile<uint32_t, RPT>(stage, tid, dst, total, pid_out, 1, 0);
+      lds_barrier();
+    }
+    if (rows_out) {
+      if (!MAPPED) {
+#pragma unroll
+        for (int k = 0; k < RPT; k++) p[k] = uint32_t(t0) + row[k];
       }
+      stage_tile<uint32_t, RPT>(stage, live, lp, MAPPED ? row : p);
+      lds_barrier();
+      store_tile<uint32_t, RPT>(stage, tid, dst, total, rows_out, 1, 0);
+      lds_barrier();
+    }
+    // the last pass moves fixed-width values straight to their place, 16-byte
+    // elements as two halves; the next loads are in flight while one is written
+    for (int c = 0, half = 0; c < nmove;) {
+      hp_move_col const mc = move[c];
+#pragma unroll
+      for (int k = 0; k < RPT; k++)  // opaque per column, as `tid`
+        asm volatile("" : "+v"(lp[k]), "+v"(dst[k]), "+v"(row[k]));
+      switch (mc.width) {
+        case 1: stage_tile<uint8_t, RPT>(stage, live, lp, raw); break;
+        case 2: stage_tile<uint16_t, RPT>(stage, live, lp, raw); break;
+        case 4: stage_tile<uint32_t, RPT>(stage, live, lp, raw); break;
+        default: stage_tile<uint64_t, RPT>(stage, live, lp, raw); break;
+      }
+      int const done = half;
+      half           = (mc.width == 16) & (half == 0);
+      c += half == 0;
+      if (c < nmove) load_moved<RPT, MAPPED>(move[c], half, t0, live, row, raw);
+      lds_barrier();
+      switch (mc.width) {
+        case 1: store_tile<uint8_t, RPT>(stage, tid, dst, total, mc.dst, 1, 0); break;
+        case 2: store_tile<uint16_t, RPT>(stage, tid, dst, total, mc.dst, 1, 0); break;
+        case 4: store_tile<uint32_t, RPT>(stage, tid, dst, total, mc.dst, 1, 0); break;
+        case 8: store_tile<uint64_t, RPT>(stage, tid, dst, total, mc.dst, 1, 0); break;
+        default: store_tile<uint64_t, RPT>(stage, tid, dst, total, mc.dst, 2, done); break;
+      }
+      lds_barrier();
     }
     if (!pid_out && !rows_out && nmove == 0) lds_barrier();  // the stage's last barrier otherwise
   }
@@ -514,13 +588,23 @@ hp_ranges hp_plan(int64_t n, int bits, int num_cus)
   return r;
 }
 
-void launch_hp_ids_count(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, bool identity,
+void launch_hp_ids_count(dcol const* d_cols, int ncols, int32_t storage, int64_t n, uint32_t seed, bool identity,
                          uint32_t num_partitions, uint32_t* pid, hp_ranges const& R, int bits, uint32_t* hist,
                          hipStream_t s)
 {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_hp_ids_count, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), sizeof(uint32_t) << bits, s, d_cols,
-                     ncols, n, seed, identity ? 1 : 0, num_partitions, pid, R.per, R.W, (1u << bits) - 1u, hist);
+  auto kernel = k_hp_ids_count<ST_NONE>;
+  if (ncols == 1 && !identity) switch (storage) {
+      case ST_I32:
+      case ST_U32: kernel = k_hp_ids_count<ST_U32>; break;
+      case ST_I64:
+      case ST_U64: kernel = k_hp_ids_count<ST_U64>; break;
+      case ST_F32: kernel = k_hp_ids_count<ST_F32>; break;
+      case ST_F64: kernel = k_hp_ids_count<ST_F64>; break;
+      default: break;
+    }
+  hipLaunchKernelGGL(kernel, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), sizeof(uint32_t) << bits, s, d_cols, ncols, n,
+                     seed, identity ? 1 : 0, num_partitions, pid, R.per, R.W, (1u << bits) - 1u, hist);
 }
 
 void launch_map_partition_ids(void const* map, int32_t map_storage, int64_t n, uint32_t num_partitions,
@@ -546,8 +630,9 @@ static void launch_scatter_form(uint32_t const* pid_in, uint32_t const* rows_in,
   constexpr size_t T = size_t(RPT) * HP_TILE_BLOCK;
   size_t const nd    = size_t(1) << bits;
   size_t const lds   = std::max(T * 8, HP_TILE_WAVES * nd * 2) + nd * 8 + T * 2;
-  hipLaunchKernelGGL(k_hp_scatter<RPT>, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), lds, s, pid_in, rows_in, n, R.per,
-                     R.W, shift, bits, start, pid_out, rows_out, move, nmove);
+  auto const kernel  = rows_in ? k_hp_scatter<RPT, true> : k_hp_scatter<RPT, false>;
+  hipLaunchKernelGGL(kernel, dim3(unsigned(R.W)), dim3(HP_TILE_BLOCK), lds, s, pid_in, rows_in, n, R.per, R.W, shift,
+                     bits, start, pid_out, rows_out, move, nmove);
 }
 
 void launch_hp_scatter(uint32_t const* pid_in, uint32_t const* rows_in, int64_t n, hp_ranges const& R, int shift,
