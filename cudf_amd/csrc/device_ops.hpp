@@ -469,6 +469,16 @@ __device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t* lds)
   return t;
 }
 
+// Workgroup barrier for phases that communicate through LDS only: each wave
+// waits for its LDS operations, not for its global stores (a __syncthreads
+// would also wait until every store of the workgroup is acknowledged).
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Address of element `i` of width `w` in an LDS byte array.
 template <typename T>
 __device__ __forceinline__ T* lds_at(uint8_t* lds, int32_t off, int64_t i)

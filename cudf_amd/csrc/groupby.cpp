@@ -47,11 +47,14 @@ constexpr int32_t RPA_LDS_BUDGET     = 80 * 1024;  // two aggregating workgroups
 constexpr int RPA_MAX_LOG_BINS       = 16;  // 256 x 256 through the two scatter passes
 constexpr int RPA_MAX_LOG_FANOUT     = 8;
 constexpr int32_t RPA_STAGE_BUDGET   = 56 * 1024;  // LDS staging of a scatter tile (3 workgroups per CU)
-// Global path, low cardinality: LDS partial tables of up to 2048 slots (3/4
-// fillable), used when the estimate is at most LDS_PREAGG_MAX_GROUPS groups.
-constexpr int32_t LDS_PREAGG_SLOTS      = 2048;
-constexpr int32_t LDS_PREAGG_MAX_GROUPS = 1024;
-constexpr int32_t LDS_PREAGG_BUDGET     = 96 * 1024;
+// Global path, low cardinality: LDS partial tables, used when the estimate is
+// at most LDS_PREAGG_MAX_GROUPS groups and their table fits; one workgroup per CU, whose 160 KB
+// also hold its 8 KB of rows that found no room.
+constexpr int32_t LDS_PREAGG_MAX_GROUPS = 4096;
+constexpr int32_t LDS_PREAGG_BUDGET     = 144 * 1024;
+// Up to this many workgroups merge their tables straight into the device-wide
+// one (a launch and the tables' copies saved: tiny calls).
+constexpr int64_t LDS_MERGE_DIRECT      = 8;
 
 // hipEvents marking phase boundaries on the call's stream.
 struct phase_timer {
@@ -645,6 +648,17 @@ class groupby_call {
   uint32_t max_mult_ = 0;  // most sampled rows sharing one key hash
   double sampled_    = 0.0;  // sampled rows the group-by keeps
   bool est_low_      = false;  // the estimate is a lower bound (skewed keys)
+  int64_t key_min_   = INT64_MAX;  // range of the sampled keys (one integer key column; else empty)
+  int64_t key_max_   = INT64_MIN;
+  uint64_t* sample_table_ = nullptr;  // hashes of the sample (launch_sample_hash)
+  uint32_t sample_mask_   = 0;
+  int64_t sample_rows_    = 0;
+  uint32_t hot_hashes_[SAMPLE_HOT_LEVELS] = {0};  // seen at least SAMPLE_HOT_MIN << j times
+  // groups that come before the partitioned path's (aggregate_hot_split), and
+  // their slots in the device-wide table
+  int64_t hot_groups_ = 0;
+  uint32_t* hot_map_  = nullptr;
+  bool split_         = false;  // the partitioned path takes the spilled rows
   // A key on at least 1/512 of the sampled rows among at most 2M groups: one
   // bin of the partitioned path would hold that key's rows (a straggler
   // workgroup), while the device-wide table of that many groups stays in the
@@ -686,7 +700,13 @@ class groupby_call {
   void gather_general_keys(uint32_t const* rep_rows, int64_t G);
   int64_t aggregate_sorted_runs();
   int64_t aggregate_partitioned();
+  int64_t aggregate_hot_split();
+  bool partitionable();
   int64_t aggregate_global();
+  int32_t lds_most_slots();
+  void lds_layout(int32_t slots);
+  size_t alloc_table(uint64_t cap);
+  void alloc_dump(int64_t blocks);
   void string_results(int64_t G);
   void finish(int64_t G);
 };
@@ -920,22 +940,43 @@ void groupby_call::estimate_groups()
     int64_t const ns = std::min<int64_t>(N, SAMPLE_ROWS);
     uint32_t const tslots = uint32_t(next_pow2(uint64_t(2 * ns)));
     auto* table    = S->get<uint64_t>(tslots);
-    auto* counters = S->get<uint32_t>(5);
+    sample_table_  = table;
+    sample_mask_   = tslots - 1;
+    sample_rows_   = ns;
+    // the key ranges, then the statistics
+    constexpr int NSTATS  = SAMPLE_STATS * SAMPLE_STAT_BLOCKS;
+    int64_t const nranges = 2 * sample_blocks(ns);
+    int32_t const kst     = P().key_storage;
+    bool const ranged     = P().key_mode == KM_INLINE && !is_float_storage(kst);
+    auto* d_ranges        = S->get<int64_t>(size_t(nranges) + (NSTATS + 1) / 2);
+    auto* d_stats         = reinterpret_cast<uint32_t*>(d_ranges + nranges);
     MIG_HIP_TRY(hipMemsetAsync(table, 0, sizeof(uint64_t) * tslots, stream_));
-    MIG_HIP_TRY(hipMemsetAsync(counters, 0, sizeof(uint32_t) * 5, stream_));
     upload(0);
-    launch_sample_hash(dP, N, ns, table, tslots - 1, counters, stream_);
-    auto* h = reinterpret_cast<uint32_t*>(pin + 2 * sizeof(gb_params));
-    MIG_HIP_TRY(hipMemcpyAsync(h, counters, 20, hipMemcpyDeviceToHost, stream_));
+    launch_sample_hash(dP, N, ns, table, tslots - 1, d_stats, ranged ? d_ranges : nullptr, stream_);
+    auto* hr = reinterpret_cast<int64_t*>(pin + 2 * sizeof(gb_params));
+    auto* h  = reinterpret_cast<uint32_t*>(hr + nranges);
+    MIG_HIP_TRY(hipMemcpyAsync(hr, d_ranges, sizeof(int64_t) * nranges + sizeof(uint32_t) * NSTATS,
+                               hipMemcpyDeviceToHost, stream_));
     MIG_HIP_TRY(hipStreamSynchronize(stream_));
-    double const sampled = double(h[0]), d = double(h[1]);
-    max_mult_ = h[2];
+    for (int64_t b = 0; ranged && b < nranges; b += 2) {
+      key_min_ = std::min(key_min_, hr[b]);
+      key_max_ = std::max(key_max_, hr[b + 1]);
+    }
+    uint32_t st[SAMPLE_STATS] = {0};
+    for (int b = 0; b < SAMPLE_STAT_BLOCKS; b++)
+      for (int j = 0; j < SAMPLE_STATS; j++) {
+        uint32_t const x = h[b * SAMPLE_STATS + j];
+        st[j]            = j == 2 ? std::max(st[j], x) : st[j] + x;
+      }
+    double const sampled = double(st[0]), d = double(st[1]);
+    max_mult_ = st[2];
     sampled_  = sampled;
+    std::copy(st + 5, st + SAMPLE_STATS, hot_hashes_);
     // population: rows that are not dropped, scaled from the sample
     pop_ = double(N) * (sampled / double(ns));
     if (ns == N) est_ = d;
     else if (sampled <= 0) est_ = 1.0;
-    else est_ = estimate_distinct_skewed(sampled, d, h[3], h[4], std::max(pop_, d), &est_low_);
+    else est_ = estimate_distinct_skewed(sampled, d, st[3], st[4], std::max(pop_, d), &est_low_);
   }
   stats_[STAT_EST_GROUPS] = est_;
 }
@@ -1251,15 +1292,11 @@ int64_t groupby_call::aggregate_sorted_runs()
   return G;
 }
 
-// Radix-partitioned LDS aggregation for high cardinality: returns the number
-// of groups, or -1 when the path does not apply (or its bins overflowed three
-// times) and the device-wide table takes the call.
-int64_t groupby_call::aggregate_partitioned()
+// Whether the partitioned path's plans hold the request.
+bool groupby_call::partitionable()
 {
-  gb_params& p    = P();
-  int const forced = g_strategy.load();
-  if (mem_ || forced == MIG_STRATEGY_GLOBAL) return -1;
-  bool rpa_ok   = !any_arg_ && (p.key_mode == KM_INLINE || p.key_mode == KM_GENERAL);
+  gb_params const& p = P();
+  bool rpa_ok = !any_arg_ && (p.key_mode == KM_INLINE || p.key_mode == KM_GENERAL);
   int n_flagged = 0;
   for (int v = 0; v < p.num_vals && rpa_ok; v++) {
     if (p.val_field_begin[v] == p.val_field_begin[v + 1]) continue;
@@ -1279,6 +1316,18 @@ int64_t groupby_call::aggregate_partitioned()
       if (p.val_field_begin[v] < p.val_field_begin[v + 1]) ncols++;
     rpa_ok = rpa_ok && ncols <= RPA_PLAN_COLS && nf_ <= RPA_PLAN_FIELDS;
   }
+  return rpa_ok;
+}
+
+// Radix-partitioned LDS aggregation for high cardinality: returns the number
+// of groups, or -1 when the path does not apply (or its bins overflowed three
+// times) and the device-wide table takes the call.
+int64_t groupby_call::aggregate_partitioned()
+{
+  gb_params& p    = P();
+  int const forced = g_strategy.load();
+  if (mem_ || forced == MIG_STRATEGY_GLOBAL) return -1;
+  bool rpa_ok = partitionable();
   // LDS of the aggregating workgroup for S hash slots: keys, S + 2 rows of
   // every accumulator, the compaction map and the shared counters.
   auto agg_lds_bytes = [&](int32_t slots, bool wide) {
@@ -1301,9 +1350,10 @@ int64_t groupby_call::aggregate_partitioned()
   bool use_rpa = false;
   if (forced == MIG_STRATEGY_PARTITIONED || forced == MIG_STRATEGY_PARTITIONED_EXACT) use_rpa = rpa_ok;
   else if (forced == MIG_STRATEGY_AUTO)  // and the estimate fits the largest partition
-    use_rpa = rpa_ok && N >= (1 << 20) && est_ >= 65536 && !heavy_hitters() &&
+    use_rpa = rpa_ok && (split_ || (N >= (1 << 20) && est_ >= 65536 && !heavy_hitters())) &&
               est_ <= double(int64_t(1) << RPA_MAX_LOG_BINS) * max_fill;
   if (!use_rpa) return -1;
+  int64_t const rows = p.num_rows;  // the input's, or those left after aggregate_hot_split
 
   int const num_cus = props().num_cus;
   rpa_params R{};
@@ -1411,7 +1461,8 @@ int64_t groupby_call::aggregate_partitioned()
   // (then the heaviest key holds under ~2e-4 of the rows with high
   // probability); a bin that still fills up is flagged and the call is
   // redone with the exact layout.
-  bool speculative = max_mult_ < 8 && pop_ >= double(1 << 20) && est_ >= 65536;
+  // the rows left by aggregate_hot_split are still skewed: laid out exactly
+  bool speculative = !split_ && max_mult_ < 8 && pop_ >= double(1 << 20) && est_ >= 65536;
   int bin_attempts = 0;
   int64_t G        = -1;
   while (G < 0 && bin_attempts < 3) {
@@ -1422,7 +1473,7 @@ int64_t groupby_call::aggregate_partitioned()
     int64_t const F1 = int64_t(1) << R.log_f1;
     int64_t const HUGE_CAP = int64_t(1) << 62;
     R.cap1 = R.cap2 = HUGE_CAP;
-    int64_t rowsA = N, rowsB = N;  // records each partition buffer holds
+    int64_t rowsA = rows, rowsB = rows;  // records each partition buffer holds
     if (speculative) {
       // rows per bin: mean mu, variance ~ mu * (1 + rows per group)
       double const m   = pop_ / std::max(est_, 1.0);
@@ -1446,18 +1497,25 @@ int64_t groupby_call::aggregate_partitioned()
     rpa_params* dR   = S->get<rpa_params>(1);
     if (!speculative) MIG_HIP_TRY(hipMemsetAsync(R.hist, 0, sizeof(uint32_t) * B, stream_));
     MIG_HIP_TRY(hipMemsetAsync(d_small, 0, sizeof(int32_t) * 4, stream_));
-    MIG_HIP_TRY(hipMemsetAsync(R.group_counter, 0, sizeof(uint64_t), stream_));
+    if (hot_groups_ > 0)
+      MIG_HIP_TRY(hipMemcpyAsync(R.group_counter, &hot_groups_, sizeof(uint64_t), hipMemcpyHostToDevice, stream_));
+    else
+      MIG_HIP_TRY(hipMemsetAsync(R.group_counter, 0, sizeof(uint64_t), stream_));
     upload(0);
     MIG_HIP_TRY(hipMemcpyAsync(dR, &R, sizeof(rpa_params), hipMemcpyHostToDevice, stream_));
     T->mark(8);
-    if (!speculative) launch_rpa_hist(dP, dR, R, N, num_cus, stream_);
+    if (!speculative) launch_rpa_hist(dP, dR, R, rows, num_cus, stream_);
     T->mark(9);
     // The output columns are allocated while the first kernels run: a bin
     // yields at most min(its rows, max_fill + 2) groups, so
     // B·(max_fill + 2) rows, and at most N, bound the groups before the bin
     // sizes are known.
-    int64_t const rows_cap = std::min<int64_t>(N, B * int64_t(max_fill + 2));
+    int64_t const rows_cap = hot_groups_ + std::min<int64_t>(rows, B * int64_t(max_fill + 2));
     alloc_outputs(rows_cap, p.key_mode == KM_GENERAL ? rows_cap : 0, true);
+    if (hot_groups_ > 0) {
+      upload(1);
+      launch_outputs(dP, p, hot_map_, hot_groups_, nullptr, stream_);
+    }
     // bin layout (starts, cursors) computed on the device
     if (speculative) launch_rpa_spec_layout(dR, R, stream_);
     else launch_rpa_layout(dR, stream_);
@@ -1510,7 +1568,7 @@ int64_t groupby_call::aggregate_partitioned()
     upload(0);
     MIG_HIP_TRY(hipMemcpyAsync(dR, &R, sizeof(rpa_params), hipMemcpyHostToDevice, stream_));
     T->mark(10);
-    launch_rpa_scatter1(dP, dR, R, N, num_cus, stream_);
+    launch_rpa_scatter1(dP, dR, R, rows, num_cus, stream_);
     T->mark(11);
     if (R.two_level) {
       launch_rpa_tiles(dR, stream_);
@@ -1564,6 +1622,186 @@ int64_t groupby_call::aggregate_partitioned()
   return G;
 }
 
+// Most slots of an LDS partial table (and of the variance pass's).
+int32_t groupby_call::lds_most_slots()
+{
+  int32_t row_bytes = 8, m2_bytes = 8;
+  for (int f = 0; f < nf_; f++) {
+    if (P().fields[f].kind == FK_M2) m2_bytes += 8;
+    else row_bytes += rpa_lds_width(P().fields[f].kind, true);  // float32 sums in float64
+  }
+  if (P().need_count_all) row_bytes += 4;
+  return (LDS_PREAGG_BUDGET / std::max(row_bytes, m2_bytes) - LDS_EXTRA_SLOTS - 16) & ~63;
+}
+
+// Lays out LDS partial tables of `slots` slots (lds_bytes stays 0 when they
+// don't fit, or the accumulators exceed the kernel's plan of one per lane).
+void groupby_call::lds_layout(int32_t slots)
+{
+  gb_params& p = P();
+  int32_t off = (slots + LDS_EXTRA_SLOTS) * 8, m2_off = off;
+  for (int f = 0; f < nf_; f++) {
+    field_desc& F = p.fields[f];
+    if (F.kind == FK_M2) {
+      p.lds_m2_off[f] = m2_off;
+      m2_off += slots * 8;
+    } else {
+      F.lds_off = off;
+      off += ((slots + LDS_EXTRA_SLOTS) * rpa_lds_width(F.kind, true) + 7) & ~7;
+    }
+  }
+  p.lds_count_off = -1;
+  if (p.need_count_all) {
+    p.lds_count_off = off;
+    off += ((slots + LDS_EXTRA_SLOTS) * 4 + 7) & ~7;
+  }
+  int32_t const bytes = std::max(off, m2_off);
+  if (bytes > LDS_PREAGG_BUDGET || nf_ > 64) return;
+  p.lds_slots = slots;
+  p.lds_fill  = slots * 17 / 20;
+  p.lds_bytes = bytes;
+}
+
+// The device-wide table of `cap` slots and its accumulators; returns their bytes.
+size_t groupby_call::alloc_table(uint64_t cap)
+{
+  gb_params& p         = P();
+  size_t state_bytes   = 0;
+  uint64_t const total = cap + 2;
+  if (p.key_mode == KM_INLINE) p.slot_keys = S->get<uint64_t>(cap);
+  else p.slot_rows = S->get<uint64_t>(cap);
+  state_bytes += 8 * cap;
+  // one array per accumulator (structure of arrays): the atomics of a
+  // row then go to different lines, which the memory system serves in
+  // parallel (a shared row of all accumulators measured slower)
+  p.slot_count   = p.need_count_all ? S->get<uint32_t>(total) : nullptr;
+  p.count_stride = 4;
+  if (p.slot_count) state_bytes += 4 * total;
+  for (int f = 0; f < nf_; f++) {
+    p.fields[f].ptr = p.fields[f].width == 8 ? static_cast<void*>(S->get<uint64_t>(total))
+                                             : static_cast<void*>(S->get<uint32_t>(total));
+    p.fields[f].stride = p.fields[f].width;
+    state_bytes += size_t(p.fields[f].width) * total;
+  }
+  return state_bytes;
+}
+
+// Room for the LDS tables of many workgroups.
+void groupby_call::alloc_dump(int64_t blocks)
+{
+  gb_params& p = P();
+  p.lds_dump   = nullptr;
+  if (blocks <= LDS_MERGE_DIRECT || mem_) return;  // a fixed arena has no room to spare
+  p.lds_dump_stride = ((p.lds_bytes + 7) & ~int64_t(7)) + 8;
+  p.lds_dump        = S->get<uint8_t>(size_t(blocks) * size_t(p.lds_dump_stride));
+}
+
+// Skewed keys: the groups of the keys seen often in the sample are aggregated
+// in LDS (they would make stragglers of their bins), and the rows of all other
+// keys become the partitioned path's input (each would cost the device-wide
+// table one atomic per accumulator, 24 G/s on this device).  No key is in
+// both, so the hot groups' results simply come first.  20M rows, Zipf(1.1) over
+// 1M values: 1.92 ms a call with LDS tables in front of the device-wide one,
+// 0.82 ms now (LDS pass 0.30, the partitioned path 0.25).  Returns the number
+// of groups, or -1 when the path does not apply.
+int64_t groupby_call::aggregate_hot_split()
+{
+  gb_params& p = P();
+  if (mem_ || g_strategy.load() != MIG_STRATEGY_AUTO || p.key_mode != KM_INLINE || any_arg_ || !heavy_hitters() ||
+      N < (1 << 20) || est_ <= double(LDS_PREAGG_MAX_GROUPS) || sample_table_ == nullptr || !partitionable())
+    return -1;
+  int32_t const slots = lds_most_slots();
+  if (slots < 1024) return -1;
+  // the fewest repeats in the sample that leave at most half the slots filled
+  int level = 0;
+  while (level < SAMPLE_HOT_LEVELS && hot_hashes_[level] > uint32_t(slots / 2)) level++;
+  if (level == SAMPLE_HOT_LEVELS || hot_hashes_[level] == 0) return -1;
+  uint32_t const at_least = uint32_t(SAMPLE_HOT_MIN) << level;
+  p.lds_bytes  = 0;
+  p.lds_direct = 0;
+  lds_layout(slots);
+  if (p.lds_bytes == 0) return -1;
+  size_t const n       = size_t(N);
+  gb_params const keep = p;  // the original columns
+  uint64_t const cap   = next_pow2(uint64_t(2 * slots));
+  int32_t* d_flags     = S->get<int32_t>(4);  // [0] overflow, [1..2] special occupancy, [3] spilled rows
+  p.cap         = cap;
+  p.cap_mask    = cap - 1;
+  p.probe_limit = uint32_t(cap);
+  p.overflow    = d_flags;
+  p.special     = reinterpret_cast<uint32_t*>(d_flags + 1);
+  p.spill_count = reinterpret_cast<uint32_t*>(d_flags + 3);
+  (void)alloc_table(cap);
+  int const blocks = props().num_cus;
+  alloc_dump(blocks);
+  p.lds_fixed = 1;
+  p.spill_key = S->get<uint8_t>(n * size_t(storage_width(p.key_storage)));
+  for (int v = 0; v < p.num_vals; v++) {
+    p.spill_val[v] = p.spill_valid[v] = nullptr;
+    if (p.val_field_begin[v] == p.val_field_begin[v + 1]) continue;
+    p.spill_val[v] = S->get<uint8_t>(n * size_t(storage_width(vals_[v].storage)));
+    if (p.vals[v].mask) p.spill_valid[v] = S->get<uint8_t>(n);
+  }
+  upload(0);
+  MIG_HIP_TRY(hipMemsetAsync(d_flags, 0, sizeof(int32_t) * 4, stream_));
+  launch_init_state(dP, p, stream_);
+  launch_insert_hot(dP, N, sample_rows_, sample_table_, sample_mask_, at_least, stream_);
+  T->mark(2);
+  launch_aggregate_lds(dP, p, blocks, stream_);
+  T->mark(3);
+  int64_t const nb       = (int64_t(cap) + 2 + SCAN_TILE - 1) / SCAN_TILE;
+  uint32_t* block_counts = S->get<uint32_t>(nb + 1);
+  launch_count_occupied(dP, p, block_counts, stream_);
+  launch_scan_blocks(block_counts, nb, block_counts + nb, stream_);
+  if (p.need_second_pass) launch_second_pass_lds(dP, p, blocks, stream_);
+  auto* h = reinterpret_cast<uint32_t*>(pin + 2 * sizeof(gb_params));
+  MIG_HIP_TRY(hipMemcpyAsync(h, d_flags, 16, hipMemcpyDeviceToHost, stream_));
+  MIG_HIP_TRY(hipMemcpyAsync(h + 4, block_counts + nb, 4, hipMemcpyDeviceToHost, stream_));
+  MIG_HIP_TRY(hipStreamSynchronize(stream_));
+  int64_t const spilled = int64_t(h[3]), hot = int64_t(h[4]);
+  double const est = est_, pop = pop_;
+  int64_t G = -1;
+  if (h[0] == 0 && spilled > 0) {
+    hot_groups_ = hot;
+    hot_map_    = S->get<uint32_t>(std::max<int64_t>(hot, 1));
+    launch_compact(dP, p, block_counts, hot_map_, stream_);
+    // the spilled rows as the input
+    p.num_rows       = spilled;
+    p.keys[0].data   = p.spill_key;
+    p.keys[0].mask   = nullptr;
+    p.skip_null_keys = 0;
+    for (int v = 0; v < p.num_vals; v++) {
+      if (!p.spill_val[v]) continue;
+      p.vals[v].data = p.spill_val[v];
+      if (!p.vals[v].mask) continue;
+      uint32_t* words = S->get<uint32_t>(size_t((spilled + 31) / 32));
+      launch_pack_valid(p.spill_valid[v], spilled, words, stream_);
+      p.vals[v].mask        = words;
+      p.vals[v].mask_offset = 0;
+    }
+    // The sample sees little of the remaining keys: at least one group per 8
+    // rows, and 4x a lower-bound estimate (bins that overflow cost a whole
+    // attempt, half-empty ones little).
+    est_      = std::max({1.0, (est_ - double(hot)) * (est_low_ ? 4.0 : 1.0), double(spilled) / 8.0});
+    est_      = std::min(est_, double(spilled));
+    pop_      = double(spilled);
+    split_    = true;
+    G         = aggregate_partitioned();
+  }
+  if (G >= 0) {  // reported as before: hot keys take the device-wide table with LDS tables in front
+    stats_[STAT_LDS_PREAGG] = 1.0;
+    stats_[STAT_STRATEGY]   = MIG_STRATEGY_GLOBAL;
+  }
+  if (G < 0) {  // back to the whole input
+    p           = keep;
+    hot_groups_ = 0;
+    split_      = false;
+    est_        = est;
+    pop_        = pop;
+  }
+  return G;
+}
+
 // The device-wide hash table (the reference's design,
 // hash/groupby.cu:548-622), growing on overflow.  Low cardinality with one
 // fixed-width key: per-workgroup LDS partial tables merged into the global
@@ -1579,38 +1817,34 @@ int64_t groupby_call::aggregate_global()
   p.lds_bytes        = 0;
   // workgroup-local tables for few groups, or for hot keys among many
   // groups (rows of keys that find no room go to the device-wide table)
-  bool const hot = heavy_hitters() && est_ > double(LDS_PREAGG_MAX_GROUPS);
-  if (p.key_mode == KM_INLINE && !any_arg_ && (est_ <= double(LDS_PREAGG_MAX_GROUPS) || hot) &&
+  if (p.key_mode == KM_INLINE && !any_arg_ && (est_ <= double(LDS_PREAGG_MAX_GROUPS) || heavy_hitters()) &&
       forced != MIG_STRATEGY_PARTITIONED) {
-    int32_t S_l = 256;
-    while (S_l < LDS_PREAGG_SLOTS && double(S_l) * 0.75 < est_ * 1.5) S_l *= 2;
-    int32_t off = S_l * 8, m2_off = S_l * 8;
-    for (int f = 0; f < nf_; f++) {
-      field_desc& F = p.fields[f];
-      if (F.kind == FK_M2) {
-        p.lds_m2_off[f] = m2_off;
-        m2_off += S_l * 8;
-      } else {
-        F.lds_off = off;
-        off += ((S_l + 2) * F.width + 7) & ~7;
-      }
+    // A third of the slots filled (the longest probe of a wave's 64 rows is
+    // what it waits for), or as many as fit: 1.2x the estimate at 85% filled
+    // is the least.  Hot keys among many groups: as many slots as fit.
+    int32_t const most  = lds_most_slots();
+    double const least  = std::max(256.0, 1.45 * est_ + 64.0);
+    bool const few      = est_ <= double(LDS_PREAGG_MAX_GROUPS) && least <= double(most);
+    bool hot            = !few && heavy_hitters() && most >= 1024;
+    int32_t S_l         = most;
+    if (few) S_l = std::min<int32_t>(most, std::max<int32_t>(256, (int32_t(3.0 * est_) + 63) & ~63));
+    // Integer keys of a range that fits (ids, dictionary codes): a slot per
+    // key of the sampled range, found without probing.
+    uint64_t const span = key_min_ <= key_max_ ? uint64_t(key_max_) - uint64_t(key_min_) : UINT64_MAX;
+    p.lds_direct        = span < uint64_t(most) && EMPTY_KEY - uint64_t(key_min_) > span + 64;
+    p.lds_key_min       = key_min_;
+    if (p.lds_direct) {
+      S_l = int32_t((span + 64) & ~uint64_t(63));
+      hot = false;
     }
-    p.lds_count_off = -1;
-    if (p.need_count_all) {
-      p.lds_count_off = off;
-      off += ((S_l + 2) * 4 + 7) & ~7;
-    }
-    int32_t const bytes = std::max(off, m2_off);
-    if (bytes <= LDS_PREAGG_BUDGET) {
-      p.lds_slots = S_l;
-      p.lds_fill  = S_l * 3 / 4;
-      p.lds_bytes = bytes;
-      int64_t const per_cu = std::max<int64_t>(1, std::min<int64_t>(8, (160 * 1024) / bytes));
-      // at least ~16 rows per group and workgroup, so that merging pays off
-      // (hot keys: the tables hold the hot keys, the rest goes through)
-      int64_t const rows_per_wg = hot ? 4096 : std::max<int64_t>(4096, int64_t(16.0 * std::max(est_, 1.0)));
-      lds_blocks = std::max<int64_t>(1, std::min<int64_t>(int64_t(num_cus) * per_cu,
-                                                           (N + rows_per_wg - 1) / rows_per_wg));
+    if (few || hot || p.lds_direct) lds_layout(S_l);
+    if (p.lds_bytes > 0) {
+      // one workgroup per CU (16 waves): more would only add tables to merge
+      // enough rows per group and workgroup that its table pays off (hot keys:
+      // the tables hold the hot keys, the rest goes through)
+      double const per_group    = mem_ ? 16.0 : 4.0;
+      int64_t const rows_per_wg = hot ? 4096 : std::max<int64_t>(4096, int64_t(per_group * std::max(est_, 1.0)));
+      lds_blocks = std::max<int64_t>(1, std::min<int64_t>(num_cus, (N + rows_per_wg - 1) / rows_per_wg));
     }
   }
   stats_[STAT_LDS_PREAGG] = lds_blocks > 0 ? 1.0 : 0.0;
@@ -1631,24 +1865,8 @@ int64_t groupby_call::aggregate_global()
                                             : std::min<uint64_t>(cap, 4096));
     p.overflow    = d_flags;
     p.special     = reinterpret_cast<uint32_t*>(d_flags + 1);
-    size_t state_bytes = 0;
-    uint64_t const total = cap + 2;
-    if (p.key_mode == KM_INLINE) p.slot_keys = S->get<uint64_t>(cap);
-    else p.slot_rows = S->get<uint64_t>(cap);
-    state_bytes += 8 * cap;
-    // one array per accumulator (structure of arrays): the atomics of a
-    // row then go to different lines, which the memory system serves in
-    // parallel (a shared row of all accumulators measured slower)
-    p.slot_count   = p.need_count_all ? S->get<uint32_t>(total) : nullptr;
-    p.count_stride = 4;
-    if (p.slot_count) state_bytes += 4 * total;
-    for (int f = 0; f < nf_; f++) {
-      p.fields[f].ptr = p.fields[f].width == 8 ? static_cast<void*>(S->get<uint64_t>(total))
-                                               : static_cast<void*>(S->get<uint32_t>(total));
-      p.fields[f].stride = p.fields[f].width;
-      state_bytes += size_t(p.fields[f].width) * total;
-    }
-    stats_[STAT_STATE_BYTES] = double(state_bytes);
+    stats_[STAT_STATE_BYTES] = double(alloc_table(cap));
+    alloc_dump(lds_blocks);
     upload(0);
     launch_init_state(dP, p, stream_);
     T->mark(2);
@@ -1809,6 +2027,10 @@ std::unique_ptr<mig_groupby_result> groupby_call::run()
   if (keys_sorted_) {
     func_range range("groupby: sorted runs");
     G = aggregate_sorted_runs();
+  }
+  if (G < 0) {
+    func_range range("groupby: hot keys apart");
+    G = aggregate_hot_split();
   }
   if (G < 0) {
     func_range range("groupby: partitioned");

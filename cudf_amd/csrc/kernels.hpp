@@ -137,6 +137,8 @@ struct out_desc {
   int32_t out_width;
 };
 
+constexpr int32_t LDS_EXTRA_SLOTS = 2 + 64;
+
 struct gb_params {
   int64_t num_rows;
   uint64_t cap;       // table slots (power of two); slots cap, cap+1 are special
@@ -167,9 +169,11 @@ struct gb_params {
   void* out_keys[MAX_KEYS];       // fixed-width key outputs (or string offsets)
   uint32_t* out_key_mask[MAX_KEYS];
   // low-cardinality pre-aggregation (inline keys): each workgroup keeps an
-  // LDS table of lds_slots keys (at most lds_fill) with partials at
-  // fields[f].lds_off (lds_slots + 2 elements of the field's width; slots
-  // lds_slots and lds_slots + 1 hold the EMPTY_KEY and null-key groups) and
+  // LDS table of lds_slots keys (at most lds_fill; lds_slots + LDS_EXTRA_SLOTS
+  // words) with partials at
+  // fields[f].lds_off (lds_slots + LDS_EXTRA_SLOTS elements of the field's
+  // width; slots lds_slots and lds_slots + 1 hold the EMPTY_KEY and null-key
+  // groups, then one slot per lane takes the rows that do not count) and
   // the row counts at lds_count_off (-1: none); the variance pass reuses the
   // bytes for a table of group slots and the M2 partials at lds_m2_off[f]
   int32_t lds_slots;
@@ -177,6 +181,22 @@ struct gb_params {
   int32_t lds_count_off;
   int32_t lds_bytes;
   int32_t lds_m2_off[MAX_FIELDS];
+  // many workgroups: each stores its table here (lds_dump_stride bytes apart,
+  // the last 8 telling which special groups it has) instead of merging it
+  uint8_t* lds_dump;
+  int64_t lds_dump_stride;
+  // integer keys of a small range: slot i is the key lds_key_min + i, and keys
+  // outside [lds_key_min, lds_key_min + lds_slots) go to the device-wide table
+  int64_t lds_key_min;
+  int32_t lds_direct;
+  // the keys of the groups kept in LDS are those in the device-wide table; the
+  // rows of all others are appended to the spill columns (element bytes, and
+  // a validity byte where the column has nulls)
+  int32_t lds_fixed;
+  uint8_t* spill_key;
+  uint8_t* spill_val[MAX_VALS];
+  uint8_t* spill_valid[MAX_VALS];
+  uint32_t* spill_count;
 };
 
 // ---------------------------------------------------------------------------
@@ -303,12 +323,28 @@ struct launch_cfg {
 
 void launch_hash_rows(dcol const* d_cols, int ncols, int64_t n, uint32_t seed, uint32_t* out,
                       hipStream_t s);
-// Distinct row hashes among `nsample` sampled rows: counters[0] = rows
-// sampled (dropped rows excluded), counters[1] = distinct hashes,
-// counters[2] = the largest number of sampled rows sharing one hash.
-// `table` has table_mask + 1 zeroed slots.
+// Row hashes of `nsample` sampled rows (dropped rows excluded): statistics of
+// the sample, one row of SAMPLE_STATS values per workgroup to be combined by
+// the caller (sums; the maximum for [2]): [0] rows sampled, [1] distinct
+// hashes, [2] the most rows sharing one hash, [3] hashes seen once, [4] twice,
+// [5 + j] hashes seen at least SAMPLE_HOT_MIN << j times.
+// `table` has table_mask + 1 zeroed slots.  `range`, for one integer key column
+// (else null), receives the smallest and largest sampled key per workgroup
+// (sample_blocks pairs; INT64_MAX, INT64_MIN where it saw none).
+constexpr int SAMPLE_HOT_MIN     = 4;
+constexpr int SAMPLE_HOT_LEVELS  = 6;
+constexpr int SAMPLE_STATS       = 5 + SAMPLE_HOT_LEVELS;
+constexpr int SAMPLE_STAT_BLOCKS = 64;
+constexpr int SAMPLE_BLOCK       = 512;
+inline int64_t sample_blocks(int64_t nsample) { return (nsample + SAMPLE_BLOCK - 1) / SAMPLE_BLOCK; }
 void launch_sample_hash(gb_params const* dP, int64_t n, int64_t nsample, uint64_t* table,
-                        uint32_t table_mask, uint32_t* counters, hipStream_t s);
+                        uint32_t table_mask, uint32_t* stats, int64_t* range, hipStream_t s);
+// Inserts the sampled keys whose hash was seen at least `at_least` times into
+// the device-wide table (inline keys; `table` as launch_sample_hash left it).
+void launch_insert_hot(gb_params const* dP, int64_t n, int64_t nsample, uint64_t const* table, uint32_t table_mask,
+                       uint32_t at_least, hipStream_t s);
+// Validity words of `n` rows from one byte per row.
+void launch_pack_valid(uint8_t const* bytes, int64_t n, uint32_t* words, hipStream_t s);
 void launch_init_state(gb_params const* dP, gb_params const& hP, hipStream_t s);
 // Allows `bytes` of dynamic LDS for kernel `fn` (above the 64 KB default;
 // gfx950 has 160 KB per CU).

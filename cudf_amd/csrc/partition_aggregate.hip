@@ -17,11 +17,10 @@
 // (groupby/hash/groupby_kernels.cuh:98-105, detail/aggregation/
 // aggregation.cuh:131-490) and its second VARIANCE pass over the whole input
 // (multi_pass_kernels.cuh:74-111), with the same results per group.
+#include "lds_accumulate.hpp"
 #include "partition_common.hpp"
 
 namespace mig {
-
-constexpr int WG_SCOPE = __HIP_MEMORY_SCOPE_WORKGROUP;
 
 constexpr int RPA_CACHED = 4;     // rows per thread per chunk; their slots stay in registers
 constexpr int RPA_OUT_BATCH = 4;  // output columns whose LDS reads are issued together
@@ -30,118 +29,6 @@ constexpr int RPA_OUT_BATCH = 4;  // output columns whose LDS reads are issued t
 // below 1e-18, so reaching it means the bin has more groups than the table
 // holds (the call is retried with more bins).
 constexpr int RPA_PROBE_LIMIT = 256;
-
-// Apply `f(k)` to the rows k of a chunk whose bit is set in `ok` (the loop is
-// unrolled; the caller's switch on the accumulator kind stays outside it).
-template <typename F>
-__device__ __forceinline__ void for_rows(uint32_t ok, F&& f)
-{
-#pragma unroll
-  for (int k = 0; k < RPA_CACHED; k++)
-    if ((ok >> k) & 1u) f(k);
-}
-
-// One accumulator over the rows of a chunk: `c[k]` holds row k's value in
-// canonical form (integers sign- or zero-extended to 64 bits, float bits
-// unchanged), `slot[k]` its group slot, bit k of `ok` whether it counts.
-__device__ __forceinline__ double canon_double(int32_t st, uint64_t c);
-
-__device__ __forceinline__ void acc_rows_lds(int32_t kind, int32_t lds_off, int32_t st, uint8_t* lds,
-                                             int const (&slot)[RPA_CACHED], uint32_t ok,
-                                             uint64_t const (&c)[RPA_CACHED], bool wide_f32)
-{
-  uint8_t* const base = lds + lds_off;
-  auto u64 = [&](int k) { return reinterpret_cast<uint64_t*>(base) + slot[k]; };
-  auto u32 = [&](int k) { return reinterpret_cast<uint32_t*>(base) + slot[k]; };
-  auto fl  = [&](int k) { return __uint_as_float(uint32_t(c[k])); };
-  auto db  = [&](int k) { return __longlong_as_double(int64_t(c[k])); };
-  constexpr int R = __ATOMIC_RELAXED;
-  switch (kind) {
-    case FK_SUM_I64: for_rows(ok, [&](int k) { __hip_atomic_fetch_add(u64(k), c[k], R, WG_SCOPE); }); break;
-    case FK_SUM_F32:  // in float64 when wide (rounded to float32 at output)
-      if (wide_f32)
-        for_rows(ok, [&](int k) {
-          __hip_atomic_fetch_add(reinterpret_cast<double*>(u64(k)), double(fl(k)), R, WG_SCOPE);
-        });
-      else
-        for_rows(ok, [&](int k) { __hip_atomic_fetch_add(reinterpret_cast<float*>(u32(k)), fl(k), R, WG_SCOPE); });
-      break;
-    case FK_SUM_F64:
-      for_rows(ok, [&](int k) { __hip_atomic_fetch_add(reinterpret_cast<double*>(u64(k)), db(k), R, WG_SCOPE); });
-      break;
-    case FK_SUMSQ_I64:
-      for_rows(ok, [&](int k) { __hip_atomic_fetch_add(u64(k), c[k] * c[k], R, WG_SCOPE); });
-      break;
-    case FK_SUMSQ_F32:
-      if (wide_f32)
-        for_rows(ok, [&](int k) {
-          double const x = double(fl(k));
-          __hip_atomic_fetch_add(reinterpret_cast<double*>(u64(k)), x * x, R, WG_SCOPE);
-        });
-      else
-        for_rows(ok, [&](int k) {
-          __hip_atomic_fetch_add(reinterpret_cast<float*>(u32(k)), fl(k) * fl(k), R, WG_SCOPE);
-        });
-      break;
-    case FK_SUMSQ_F64:
-      for_rows(ok, [&](int k) {
-        __hip_atomic_fetch_add(reinterpret_cast<double*>(u64(k)), db(k) * db(k), R, WG_SCOPE);
-      });
-      break;
-    case FK_MIN_S32:
-      for_rows(ok, [&](int k) {
-        __hip_atomic_fetch_min(reinterpret_cast<int32_t*>(u32(k)), int32_t(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_MAX_S32:
-      for_rows(ok, [&](int k) {
-        __hip_atomic_fetch_max(reinterpret_cast<int32_t*>(u32(k)), int32_t(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_MIN_S64:
-      for_rows(ok, [&](int k) {
-        __hip_atomic_fetch_min(reinterpret_cast<int64_t*>(u64(k)), int64_t(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_MAX_S64:
-      for_rows(ok, [&](int k) {
-        __hip_atomic_fetch_max(reinterpret_cast<int64_t*>(u64(k)), int64_t(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_MIN_U32: for_rows(ok, [&](int k) { __hip_atomic_fetch_min(u32(k), uint32_t(c[k]), R, WG_SCOPE); }); break;
-    case FK_MAX_U32: for_rows(ok, [&](int k) { __hip_atomic_fetch_max(u32(k), uint32_t(c[k]), R, WG_SCOPE); }); break;
-    case FK_MIN_U64: for_rows(ok, [&](int k) { __hip_atomic_fetch_min(u64(k), c[k], R, WG_SCOPE); }); break;
-    case FK_MAX_U64: for_rows(ok, [&](int k) { __hip_atomic_fetch_max(u64(k), c[k], R, WG_SCOPE); }); break;
-    case FK_MIN_F32:
-      for_rows(ok, [&](int k) {
-        if (!isnan(fl(k))) __hip_atomic_fetch_min(u32(k), ord32(uint32_t(c[k])), R, WG_SCOPE);
-      });
-      break;
-    case FK_MAX_F32:
-      for_rows(ok, [&](int k) {
-        if (!isnan(fl(k))) __hip_atomic_fetch_max(u32(k), ord32(uint32_t(c[k])), R, WG_SCOPE);
-      });
-      break;
-    case FK_MIN_F64:
-      for_rows(ok, [&](int k) {
-        if (!isnan(db(k))) __hip_atomic_fetch_min(u64(k), ord64(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_MAX_F64:
-      for_rows(ok, [&](int k) {
-        if (!isnan(db(k))) __hip_atomic_fetch_max(u64(k), ord64(c[k]), R, WG_SCOPE);
-      });
-      break;
-    case FK_COUNT: for_rows(ok, [&](int k) { __hip_atomic_fetch_add(u32(k), 1u, R, WG_SCOPE); }); break;
-    case FK_M2:  // pass A: sum of squares in double (finalised into M2 after the pass)
-      for_rows(ok, [&](int k) {
-        double const x = canon_double(st, c[k]);
-        __hip_atomic_fetch_add(reinterpret_cast<double*>(u64(k)), x * x, R, WG_SCOPE);
-      });
-      break;
-    default: break;
-  }
-}
 
 __device__ __forceinline__ double lds_field_double(field_desc const& F, uint8_t* lds, int id, bool wide_f32)
 {
@@ -199,64 +86,6 @@ struct rpa_misc {
   uint32_t wave_sum[RPA_AGG_BLOCK / 64];
 };
 
-// Raw elements of a partition value column for the rows [r0 + k * block)
-// of a chunk, zero-extended to 64 bits (canon_rows gives the canonical form).
-// Rows past the bin read its last row; their lanes take no part.
-template <typename T>
-__device__ __forceinline__ void load_rows(gmem<T const>* p, int64_t r0, int64_t e, uint64_t (&c)[RPA_CACHED])
-{
-#pragma unroll
-  for (int k = 0; k < RPA_CACHED; k++) {
-    int64_t const r = r0 + int64_t(k) * RPA_AGG_BLOCK;
-    c[k]            = uint64_t(p[r < e ? r : e - 1]);
-  }
-}
-
-__device__ __forceinline__ void load_chunk(gmem<uint8_t const>* src, int w, int64_t r0, int64_t e,
-                                           uint64_t (&c)[RPA_CACHED])
-{
-  switch (w) {
-    case 1: load_rows(src, r0, e, c); break;
-    case 2: load_rows(reinterpret_cast<gmem<uint16_t const>*>(src), r0, e, c); break;
-    case 4: load_rows(reinterpret_cast<gmem<uint32_t const>*>(src), r0, e, c); break;
-    default: load_rows(reinterpret_cast<gmem<uint64_t const>*>(src), r0, e, c); break;
-  }
-}
-
-// Canonical form of a chunk's raw elements of storage `st`: integers sign-
-// or zero-extended to 64 bits (bool as 0/1), float bits unchanged.
-__device__ __forceinline__ void canon_rows(int32_t st, uint64_t (&c)[RPA_CACHED])
-{
-  switch (st) {
-    case ST_I8:
-#pragma unroll
-      for (int k = 0; k < RPA_CACHED; k++) c[k] = uint64_t(int64_t(int8_t(c[k])));
-      break;
-    case ST_I16:
-#pragma unroll
-      for (int k = 0; k < RPA_CACHED; k++) c[k] = uint64_t(int64_t(int16_t(c[k])));
-      break;
-    case ST_I32:
-#pragma unroll
-      for (int k = 0; k < RPA_CACHED; k++) c[k] = uint64_t(int64_t(int32_t(c[k])));
-      break;
-    case ST_BOOL:
-#pragma unroll
-      for (int k = 0; k < RPA_CACHED; k++) c[k] = c[k] != 0;
-      break;
-    default: break;
-  }
-}
-
-// A canonical element as double.
-__device__ __forceinline__ double canon_double(int32_t st, uint64_t c)
-{
-  if (st == ST_F64) return __longlong_as_double(int64_t(c));
-  if (st == ST_F32) return double(__uint_as_float(uint32_t(c)));
-  if (st == ST_U64) return double(c);
-  return double(int64_t(c));
-}
-
 // What pass A needs of the request, held in registers for the whole bin.
 // Every load from the kernel parameters is a scalar memory read, and waiting
 // for one also waits for all LDS operations in flight (one counter covers
@@ -302,15 +131,11 @@ __device__ __forceinline__ acc_plan load_plan(gb_params const& P, rpa_params con
   return A;
 }
 
-__device__ __forceinline__ uint32_t lane_value(uint32_t v, int i)
-{
-  return uint32_t(__builtin_amdgcn_readlane(int(v), i));
-}
-
 // Raw values of the first RPA_AGG_PREFETCH value columns of a chunk, loaded
 // together with the chunk's keys and flags so that the chunk waits for memory
 // once, not once per column.
-constexpr int RPA_AGG_PREFETCH = 1;
+// (100M rows, two columns: one column 1,761 us, two 1,700 us.)
+constexpr int RPA_AGG_PREFETCH = 2;
 struct chunk_prefetch {
   uint64_t c[RPA_AGG_PREFETCH][RPA_CACHED];
 };
@@ -341,7 +166,7 @@ __device__ __forceinline__ void prefetch_values(acc_plan const& A, int64_t r0, i
   for (int i = 0; i < RPA_AGG_PREFETCH; i++) {
     if (i >= A.ncols) break;
     uint32_t const cd = lane_value(A.cd_lane, i);
-    load_chunk(plan_column(A, i), storage_width(int(cd & 0xffu)), r0, e, pf.c[i]);
+    load_chunk<RPA_AGG_BLOCK>(plan_column(A, i), storage_width(int(cd & 0xffu)), r0, e, pf.c[i]);
   }
 }
 
@@ -486,7 +311,7 @@ __device__ __forceinline__ void chunk_accumulate(acc_plan const& A, uint8_t* lds
 #pragma unroll
   for (int k = 0; k < RPA_CACHED; k++) live |= uint32_t(slot[k] >= 0) << k;
   if (A.count_all_off >= 0)
-    for_rows(live, [&](int k) {
+    for_rows<RPA_CACHED>(live, [&](int k) {
       __hip_atomic_fetch_add(lds_at<uint32_t>(lds, A.count_all_off, slot[k]), 1u, __ATOMIC_RELAXED, WG_SCOPE);
     });
   auto column = [&](int i, uint64_t (&c)[RPA_CACHED]) {
@@ -501,9 +326,13 @@ __device__ __forceinline__ void chunk_accumulate(acc_plan const& A, uint8_t* lds
 #pragma unroll
       for (int k = 0; k < RPA_CACHED; k++) ok &= ~(uint32_t(((flp >> (8 * k + bit)) & 1) == 0) << k);
     }
+    int at[RPA_CACHED];
+#pragma unroll
+    for (int k = 0; k < RPA_CACHED; k++) at[k] = slot[k];
     for (int f = fb; f < fe; f++) {
       uint32_t const d = lane_value(A.fd_lane, f);
-      acc_rows_lds(int32_t(d & 0xffu), int32_t(d >> 8), st, lds, slot, ok, c, A.wide_f32);
+      opaque_rows(at, c);
+      acc_rows_lds(int32_t(d & 0xffu), int32_t(d >> 8), st, lds, at, ok, c, A.wide_f32);
     }
   };
 #pragma unroll
@@ -516,7 +345,7 @@ __device__ __forceinline__ void chunk_accumulate(acc_plan const& A, uint8_t* lds
   }
   for (int i = RPA_AGG_PREFETCH; i < A.ncols; i++) {
     uint64_t c[RPA_CACHED];
-    load_chunk(plan_column(A, i), storage_width(int(lane_value(A.cd_lane, i) & 0xffu)), r0, e, c);
+    load_chunk<RPA_AGG_BLOCK>(plan_column(A, i), storage_width(int(lane_value(A.cd_lane, i) & 0xffu)), r0, e, c);
     column(i, c);
   }
 }
@@ -545,14 +374,14 @@ __device__ __forceinline__ void chunk_deviations(gb_params const& P, rpa_params 
     int const w         = storage_width(st);
     field_desc const& F = P.fields[m2];
     uint64_t c[RPA_CACHED];
-    load_chunk(gp(static_cast<uint8_t const*>(R.valsB[v])), w, r0, e, c);
+    load_chunk<RPA_AGG_BLOCK>(gp(static_cast<uint8_t const*>(R.valsB[v])), w, r0, e, c);
     canon_rows(st, c);
     uint32_t ok = live;
     if (bit >= 0) {
 #pragma unroll
       for (int k = 0; k < RPA_CACHED; k++) ok &= ~(uint32_t(((flp >> (8 * k + bit)) & 1) == 0) << k);
     }
-    for_rows(ok & flagged, [&](int k) {
+    for_rows<RPA_CACHED>(ok & flagged, [&](int k) {
       double const x    = canon_double(st, c[k]);
       double const cnt  = double(lds_count(P, R, lds, F.aux_count, slot[k]));
       double const mean = lds_field_double(P.fields[F.aux_sum], lds, slot[k], R.wide_f32 != 0) / cnt;

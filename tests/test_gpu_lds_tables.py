@@ -1,0 +1,88 @@
+"""Workgroup-local tables of the hash group-by against the CPU oracle: slots
+taken by the key's value, tables that many workgroups store and merge, and the
+split of hot keys from the partitioned path.  Integer results are compared
+exactly, floating sums within the parity helper's bound (sums in another order)."""
+import numpy as np
+import pytest
+
+from tests.gbutil import AGG, C2_AGGS, assert_parity, host_col
+
+pytestmark = pytest.mark.gpu
+
+SENTINEL = np.array([0xFFF1A5A5A5A5A5A5], dtype=np.uint64)  # the tables' empty marker
+
+
+def _stats():
+    from cudf_amd import _lib
+    return _lib.last_stats()
+
+
+@pytest.mark.parametrize("dtype,low,card,n", [
+    (np.int8, -128, 256, 300_000),            # negative keys of a narrow type
+    (np.bool_, 0, 2, 20_000),
+    (np.uint16, 65_000, 536, 70_001),
+    (np.int32, -2**31, 1_000, 1_200_000),     # the type's smallest values
+    (np.uint32, 2**32 - 700, 700, 600_001),
+    (np.int64, 2**63 - 1_500, 1_500, 900_000),  # the type's largest
+    (np.uint64, 2**63 - 20, 64, 50_000),      # across the sign bit
+    (np.int64, int(SENTINEL.view(np.int64)[0]) - 30, 64, 50_000),  # around the empty marker: probed
+])
+@pytest.mark.parametrize("policy", [0, 1])
+def test_keys_of_a_small_range(dtype, low, card, n, policy):
+    rng = np.random.default_rng(n + policy)
+    k = (rng.integers(0, card, n).astype(object) + low) if card > 2 else rng.integers(0, 2, n)
+    k = np.array(k, dtype=dtype)
+    key = host_col(k, rng.random(n) >= 0.02)
+    f = host_col(rng.standard_normal(n).astype(np.float32), rng.random(n) >= 0.05)
+    i = host_col(rng.integers(-1000, 1000, n))
+    assert_parity([key], [(f, [(AGG["SUM"], 1), (AGG["MAX"], 1), (AGG["COUNT_VALID"], 1)]),
+                          (i, [(AGG["SUM"], 1), (AGG["MIN"], 1), (AGG["MEAN"], 1), (AGG["COUNT_ALL"], 1)])], policy)
+    assert _stats()["lds_preagg"] == 1.0
+
+
+@pytest.mark.parametrize("n", [40_000, 1_500_000])
+def test_keys_outside_the_sampled_range(n):
+    """A few rows hold keys far from the others: whether the sample sees them
+    or not, they get groups of their own."""
+    rng = np.random.default_rng(n)
+    k = rng.integers(0, 500, n)
+    far = rng.choice(n, 40, replace=False)
+    k[far] = 10**12 + rng.integers(0, 20, 40)
+    v = host_col(rng.integers(-100, 100, n))
+    assert_parity([host_col(k)], [(v, [(AGG["SUM"], 1), (AGG["MIN"], 1), (AGG["COUNT_ALL"], 1)])])
+
+
+@pytest.mark.parametrize("card", [1, 63, 2_300, 4_000, 4_097])
+def test_sparse_keys_and_special_floats(card):
+    """Keys without a small range (probed tables, up to and past what LDS
+    holds), values with NaN and infinities."""
+    rng = np.random.default_rng(card)
+    n = 400_003
+    k = rng.integers(-2**62, 2**62, card)[rng.integers(0, card, n)]
+    x = rng.standard_normal(n)
+    x[rng.integers(0, n, 300)] = np.nan
+    x[rng.integers(0, n, 30)] = np.inf
+    f = host_col(x, rng.random(n) >= 0.1)
+    assert_parity([host_col(k)], [(f, [(AGG["MIN"], 1), (AGG["MAX"], 1), (AGG["COUNT_VALID"], 1)]),
+                                  (host_col(rng.integers(0, 9, n).astype(np.uint8)), [(AGG["SUM"], 1), (AGG["MAX"], 1)])])
+
+
+@pytest.mark.parametrize("key_dtype,policy,nulls", [(np.int64, 0, 0.0), (np.int64, 1, 0.05), (np.int32, 1, 0.05),
+                                                    (np.float64, 0, 0.05)])
+def test_hot_keys_apart_from_the_rest(key_dtype, policy, nulls):
+    """A third of the rows on 40 keys, the others on 300,000 more: the hot
+    groups and the partitioned path's make one result, with every aggregation
+    of both kinds of pass."""
+    rng = np.random.default_rng(11)
+    n = 1_300_007
+    k = rng.integers(0, 300_000, n)
+    hot = rng.random(n) < 0.34
+    k[hot] = rng.integers(0, 40, int(hot.sum())) * 7
+    k = k.astype(key_dtype)
+    if key_dtype == np.int64:
+        k[rng.integers(0, n, 5_000)] = SENTINEL.view(np.int64)[0]
+    key = host_col(k, rng.random(n) >= nulls if nulls else None)
+    f = host_col(rng.standard_normal(n) * 10 + 3, rng.random(n) >= nulls if nulls else None)
+    i = host_col(rng.integers(0, 10_000, n).astype(np.int32), rng.random(n) >= 0.03)
+    assert_parity([key], [(f, C2_AGGS), (i, C2_AGGS)], policy)
+    assert _stats()["lds_preagg"] == 1.0 and _stats()["strategy"] == 1
