@@ -431,6 +431,17 @@ void launch_sorted_string_arg(gb_params const* dP, gb_params const& hP, int64_t 
 // rows[g] = perm[rows[g]] where rows[g] >= 0.
 void launch_map_rows(int32_t* rows, int64_t G, uint32_t const* perm, hipStream_t s);
 
+// Sorting inside groups for the quantiles: rows `perm` in group order with the
+// groups at off[0..G].  launch_list_groups collects the groups a wave's
+// registers don't hold (`list`, counts[0]; counts zeroed by the caller) and
+// sets counts[1] when one has more than SORT_BLOCK_ROWS rows; if none has,
+// launch_sort_groups writes every group's values, as order-preserving bits
+// (`hi` for 8-byte values), ascending with nulls (`nul`, may be null) last.
+constexpr int SORT_BLOCK_ROWS = 8192;
+void launch_list_groups(int32_t const* off, int64_t G, uint32_t* list, uint32_t* counts, hipStream_t s);
+void launch_sort_groups(dcol const& v, uint32_t const* perm, int32_t const* off, int64_t G, uint32_t const* list,
+                        int64_t listed, uint32_t* lo, uint32_t* hi, uint32_t* nul, hipStream_t s);
+
 // ---- sort-based aggregations (sort_kernels.hip, label kernels in
 // groupby_kernels.hip) ---------------------------------------------------------
 // Every row's slot in the device-wide table (inserting its key), UINT32_MAX

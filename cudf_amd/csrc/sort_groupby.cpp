@@ -164,6 +164,19 @@ std::unique_ptr<mig_groupby_result> sort_groupby(mig_column_view const* keys, in
   launch_hp_offsets(gid_sorted, N, uint32_t(G + 2), off, stream);
   int32_t kept = 0;
   MIG_HIP_TRY(hipMemcpyAsync(&kept, off + G, 4, hipMemcpyDeviceToHost, stream));
+  // the groups too long for a wave, when quantiles need sorted values
+  bool quantiles = false;
+  for (int r = 0; r < num_requests; r++)
+    for (int a = 0; a < requests[r].num_aggregations; a++) quantiles |= is_sort_only(requests[r].aggregations[a].kind);
+  uint32_t* long_groups    = nullptr;
+  uint32_t long_counts[2] = {0, 0};
+  if (quantiles) {
+    long_groups      = S.get<uint32_t>(std::max<int64_t>(G, 1));
+    uint32_t* counts = S.get<uint32_t>(2);
+    MIG_HIP_TRY(hipMemsetAsync(counts, 0, 8, stream));
+    launch_list_groups(off, G, long_groups, counts, stream);
+    MIG_HIP_TRY(hipMemcpyAsync(long_counts, counts, 8, hipMemcpyDeviceToHost, stream));
+  }
   MIG_HIP_TRY(hipStreamSynchronize(stream));
 
   // ---- 3. the other aggregations on the rows in group order ---------------------
@@ -270,6 +283,14 @@ std::unique_ptr<mig_groupby_result> sort_groupby(mig_column_view const* keys, in
     bool const wide   = storage_width(st) == 8;
     bool const nulls  = v.null_mask && null_count_of(v, stream) > 0;
     dcol const dv     = make_dcol(v, nulls);
+    if (long_counts[1] == 0) {  // every group fits a workgroup
+      size_t const n = size_t(std::max(kept, 1));
+      sorted_values const out{v, S.get<uint32_t>(n), wide ? S.get<uint32_t>(n) : nullptr,
+                              nulls ? S.get<uint32_t>(n) : nullptr};
+      launch_sort_groups(dv, perm, off, G, long_groups, int64_t(long_counts[0]), out.lo, out.hi, out.nul, stream);
+      sorted.push_back(out);
+      return out;
+    }
     uint32_t* lo      = S.get<uint32_t>(N);
     uint32_t* hi      = wide ? S.get<uint32_t>(N) : nullptr;
     uint32_t* nul     = nulls ? S.get<uint32_t>(N) : nullptr;

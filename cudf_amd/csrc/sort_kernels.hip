@@ -3,10 +3,13 @@
 // The reference sorts the keys, then sorts each group's values and reads the
 // quantiles off the sorted segments (sort/sort_helper.cu, sort/
 // group_quantiles.cu:30-80, quantiles/quantiles_util.hpp).  Here the rows are
-// labelled with their group by the hash table, and one stable LSD counting
-// sort orders them by (group, null, value) using the order-preserving bits
-// written by k_quantile_keys; k_group_quantiles then reads every group's
-// segment.
+// labelled with their group by the hash table and brought into group order by
+// a stable LSD counting sort of the group numbers.  The values' order-
+// preserving bits are then sorted group by group on the chip
+// (k_sort_groups_wave, k_sort_groups_block) while every group has at most
+// SORT_BLOCK_ROWS rows, else by more passes of the counting sort, over (group,
+// null, value) with the bits written by k_quantile_keys.  k_group_quantiles
+// reads every group's segment.
 #include "device_ops.hpp"
 #include "kernels.hpp"
 
@@ -63,6 +66,221 @@ __global__ void __launch_bounds__(SBLOCK)
   gp(lo)[r]        = uint32_t(o);
   if (hi) gp(hi)[r] = uint32_t(o >> 32);
   if (null_flag) gp(null_flag)[r] = valid ? 0u : 1u;
+}
+
+// ---------------------------------------------------------------------------
+// Sorting inside groups.  Nine counting passes (64-bit values, nulls, group)
+// over 4M rows in 50,000 groups took 1.3 ms; gathering the order bits and
+// sorting each group where it is held takes 0.07 ms (a call
+// with MEDIAN, MAX and NUNIQUE 2.45 -> 1.43 ms).
+
+// The value of lane (own lane ^ d), d a power of two.
+__device__ __forceinline__ uint64_t lane_xor(uint64_t x, int d)
+{
+  uint32_t const lo = uint32_t(x), hi = uint32_t(x >> 32);
+  switch (d) {  // constants after unrolling; DPP where it has the pattern
+    case 1:
+      return (uint64_t(uint32_t(__builtin_amdgcn_mov_dpp(int(hi), 0xB1, 0xF, 0xF, true))) << 32) |
+             uint32_t(__builtin_amdgcn_mov_dpp(int(lo), 0xB1, 0xF, 0xF, true));
+    case 2:
+      return (uint64_t(uint32_t(__builtin_amdgcn_mov_dpp(int(hi), 0x4E, 0xF, 0xF, true))) << 32) |
+             uint32_t(__builtin_amdgcn_mov_dpp(int(lo), 0x4E, 0xF, 0xF, true));
+    case 8:
+      return (uint64_t(uint32_t(__builtin_amdgcn_mov_dpp(int(hi), 0x128, 0xF, 0xF, true))) << 32) |
+             uint32_t(__builtin_amdgcn_mov_dpp(int(lo), 0x128, 0xF, 0xF, true));
+    default: return (uint64_t(uint32_t(__shfl_xor(int(hi), d, 64))) << 32) | uint32_t(__shfl_xor(int(lo), d, 64));
+  }
+}
+
+// Bitonic sort of a wave's 64 * R values, element lane * R + r in v[r], so
+// that steps of distance below R stay inside a lane; descending when `down`.
+template <int R>
+__device__ __forceinline__ void wave_sort(uint64_t (&v)[R], bool down)
+{
+  int const lane = int(threadIdx.x & 63u);
+#pragma unroll
+  for (int k = 2; k <= 64 * R; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        // the block of k elements is ascending (the last one: as asked)
+        bool const up = k == 64 * R ? !down : (k < R ? (r & k) == 0 : (lane & (k / R)) == 0);
+        if (j < R) {
+          if (r & j) continue;
+          uint64_t const a = v[r], b = v[r | j];
+          bool const swap  = up ? b < a : a < b;
+          v[r]             = swap ? b : a;
+          v[r | j]         = swap ? a : b;
+        } else {
+          uint64_t const o    = lane_xor(v[r], j / R);
+          bool const keep_min = ((lane & (j / R)) == 0) == up;
+          v[r]                = (o < v[r]) == keep_min ? o : v[r];
+        }
+      }
+    }
+  }
+}
+
+// The last steps of a bitonic merge, inside 64 * R values with element
+// r * 64 + lane in v[r].
+template <int R>
+__device__ __forceinline__ void wave_merge(uint64_t (&v)[R], bool down)
+{
+  int const lane = int(threadIdx.x & 63u);
+#pragma unroll
+  for (int j = 32 * R; j > 0; j >>= 1) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      if (j >= 64) {
+        if (r & (j / 64)) continue;
+        uint64_t const a = v[r], b = v[r | (j / 64)];
+        bool const swap  = down ? a < b : b < a;
+        v[r]             = swap ? b : a;
+        v[r | (j / 64)]  = swap ? a : b;
+      } else {
+        uint64_t const o    = lane_xor(v[r], j);
+        bool const keep_min = ((lane & j) == 0) != down;
+        v[r]                = (o < v[r]) == keep_min ? o : v[r];
+      }
+    }
+  }
+}
+
+// Order bits of the rows at places [b, e) of the group order; nulls and places
+// past the end take the largest value, so that the first `valid` sorted places
+// hold the valid values (equal bits are equal values).
+struct group_sort {
+  dcol v;
+  uint32_t const* perm;
+  uint32_t* lo;
+  uint32_t* hi;   // 8-byte values
+  uint32_t* nul;  // null flags, or nullptr when the column has no nulls
+};
+
+__device__ __forceinline__ uint64_t group_value(group_sort const& J, int64_t at, int64_t e, uint32_t& valid)
+{
+  bool ok    = at < e;
+  uint64_t o = ~0ull;
+  if (ok) {
+    int64_t const row = gp(J.perm)[at];
+    ok                = dcol_valid(J.v, row);
+    if (ok) o = order_bits(J.v, row);
+  }
+  valid += uint32_t(__popcll(__builtin_amdgcn_ballot_w64(ok)));
+  return o;
+}
+
+__device__ __forceinline__ void group_store(group_sort const& J, int64_t at, int64_t e, uint64_t o, bool null)
+{
+  if (at >= e) return;
+  gp(J.lo)[at] = uint32_t(o);
+  if (J.hi) gp(J.hi)[at] = uint32_t(o >> 32);
+  if (J.nul) gp(J.nul)[at] = null ? 1u : 0u;
+}
+
+constexpr int SORT_WAVE_ROWS = 512;  // a wave's registers hold 8 values per lane
+
+template <int R>
+__device__ __forceinline__ void sort_group(group_sort const& J, int64_t b, int64_t e)
+{
+  int const lane = int(threadIdx.x & 63u);
+  uint64_t v[R];
+  uint32_t valid = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) v[r] = group_value(J, b + r * 64 + lane, e, valid);
+  wave_sort<R>(v, false);
+#pragma unroll
+  for (int r = 0; r < R; r++) group_store(J, b + lane * R + r, e, v[r], uint32_t(lane * R + r) >= valid);
+}
+
+// One wave per group of at most SORT_WAVE_ROWS rows.
+__global__ void __launch_bounds__(SBLOCK) k_sort_groups_wave(group_sort J, int32_t const* __restrict__ off, int64_t G)
+{
+  int64_t const g = int64_t(blockIdx.x) * (SBLOCK / 64) + (threadIdx.x >> 6);
+  if (g >= G) return;
+  int64_t const b = gp(off)[g], e = gp(off)[g + 1];
+  int64_t const n = e - b;
+  if (n <= 64) sort_group<1>(J, b, e);
+  else if (n <= 128) sort_group<2>(J, b, e);
+  else if (n <= 256) sort_group<4>(J, b, e);
+  else if (n <= SORT_WAVE_ROWS) sort_group<8>(J, b, e);
+}
+
+// One workgroup per listed group (up to SORT_BLOCK_ROWS rows): chunks of
+// SORT_WAVE_ROWS sorted in registers, alternately up and down, then merged;
+// only the steps across chunks go through LDS.
+constexpr int SORT_BLOCK = 512;
+
+__global__ void __launch_bounds__(SORT_BLOCK)
+  k_sort_groups_block(group_sort J, int32_t const* __restrict__ off, uint32_t const* __restrict__ list)
+{
+  __shared__ uint64_t x[SORT_BLOCK_ROWS];
+  __shared__ uint32_t valid_sh;
+  constexpr int R = SORT_WAVE_ROWS / 64;
+  int64_t const g = gp(list)[blockIdx.x];
+  int64_t const b = gp(off)[g], e = gp(off)[g + 1];
+  int size = 2 * SORT_WAVE_ROWS;
+  while (size < int(e - b)) size *= 2;
+  int const chunks = size / SORT_WAVE_ROWS, wave = int(threadIdx.x >> 6), lane = int(threadIdx.x & 63u);
+  if (threadIdx.x == 0) valid_sh = 0;
+  __syncthreads();
+  uint32_t valid = 0;
+  for (int c = wave; c < chunks; c += SORT_BLOCK / 64) {
+    uint64_t v[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) v[r] = group_value(J, b + c * SORT_WAVE_ROWS + r * 64 + lane, e, valid);
+    wave_sort<R>(v, (c & 1) != 0);
+#pragma unroll
+    for (int r = 0; r < R; r++) x[c * SORT_WAVE_ROWS + lane * R + r] = v[r];
+  }
+  if (lane == 0) __hip_atomic_fetch_add(&valid_sh, valid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __syncthreads();
+  valid = valid_sh;
+  for (int k = 2 * SORT_WAVE_ROWS; k <= size; k *= 2) {
+    for (int j = k / 2; j >= SORT_WAVE_ROWS; j /= 2) {
+      for (int i = threadIdx.x; i < size / 2; i += SORT_BLOCK) {
+        int const at     = ((i & ~(j - 1)) << 1) | (i & (j - 1));
+        uint64_t const p = x[at], q = x[at + j];
+        if (((at & k) == 0) == (q < p)) {
+          x[at]     = q;
+          x[at + j] = p;
+        }
+      }
+      __syncthreads();
+    }
+    for (int c = wave; c < chunks; c += SORT_BLOCK / 64) {
+      uint64_t v[R];
+      int const c0 = c * SORT_WAVE_ROWS;
+#pragma unroll
+      for (int r = 0; r < R; r++) v[r] = x[c0 + r * 64 + lane];
+      wave_merge<R>(v, (c0 & k) != 0);
+      if (k < size) {
+#pragma unroll
+        for (int r = 0; r < R; r++) x[c0 + r * 64 + lane] = v[r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          int const i = c0 + r * 64 + lane;
+          group_store(J, b + i, e, v[r], uint32_t(i) >= valid);
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Groups by how they are sorted: counts[0] listed ones (more than
+// SORT_WAVE_ROWS rows), counts[1] those past SORT_BLOCK_ROWS.
+__global__ void __launch_bounds__(SBLOCK)
+  k_list_groups(int32_t const* __restrict__ off, int64_t G, uint32_t* __restrict__ list, uint32_t* counts)
+{
+  int64_t const g = int64_t(blockIdx.x) * SBLOCK + threadIdx.x;
+  if (g >= G) return;
+  int32_t const n = gp(off)[g + 1] - gp(off)[g];
+  if (n <= SORT_WAVE_ROWS) return;
+  if (n > SORT_BLOCK_ROWS) astore(counts + 1, 1u);
+  gp(list)[__hip_atomic_fetch_add(gp(counts), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)] = uint32_t(g);
 }
 
 // The element of storage `st` whose order bits are (lo, hi), as double.
@@ -179,6 +397,20 @@ int64_t sgrid(int64_t n) { return (n + SBLOCK - 1) / SBLOCK; }
 void launch_quantile_keys(dcol const& v, int64_t n, uint32_t* lo, uint32_t* hi, uint32_t* null_flag, hipStream_t s)
 {
   if (n > 0) hipLaunchKernelGGL(k_quantile_keys, dim3(sgrid(n)), dim3(SBLOCK), 0, s, v, n, lo, hi, null_flag);
+}
+
+void launch_list_groups(int32_t const* off, int64_t G, uint32_t* list, uint32_t* counts, hipStream_t s)
+{
+  if (G > 0) hipLaunchKernelGGL(k_list_groups, dim3(sgrid(G)), dim3(SBLOCK), 0, s, off, G, list, counts);
+}
+
+void launch_sort_groups(dcol const& v, uint32_t const* perm, int32_t const* off, int64_t G, uint32_t const* list,
+                        int64_t listed, uint32_t* lo, uint32_t* hi, uint32_t* nul, hipStream_t s)
+{
+  if (G <= 0) return;
+  group_sort const J{v, perm, lo, hi, nul};
+  hipLaunchKernelGGL(k_sort_groups_wave, dim3((G + SBLOCK / 64 - 1) / (SBLOCK / 64)), dim3(SBLOCK), 0, s, J, off, G);
+  if (listed > 0) hipLaunchKernelGGL(k_sort_groups_block, dim3(listed), dim3(SORT_BLOCK), 0, s, J, off, list);
 }
 
 void launch_group_quantiles(uint32_t const* ord_lo, uint32_t const* ord_hi, uint32_t const* null_flag,
