@@ -152,6 +152,10 @@ SIGNATURES = {
     "mig_batch_execute": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),
     "mig_batch_synchronize": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),
     "mig_batch_num_groups": (ctypes.c_int32, [ctypes.c_void_p, ctypes.c_int32]),
+    "mig_batch_result": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.POINTER(OutColumn),
+                                        ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
+                                        ctypes.POINTER(ctypes.c_int64)]),
+    "mig_batch_result_copy": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]),
     "mig_batch_result_key": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.POINTER(OutColumn)]),
     "mig_batch_result_column": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32,
                                                ctypes.c_int32, ctypes.POINTER(OutColumn)]),

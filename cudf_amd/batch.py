@@ -43,23 +43,6 @@ def _stream_handle(stream: Optional[torch.cuda.Stream]):
     return ctypes.c_void_p(s.cuda_stream)
 
 
-class _DeviceBytes:
-    """A borrowed device byte range, exposed to torch through the CUDA array
-    interface (a zero-copy view that torch then copies)."""
-
-    def __init__(self, ptr: int, nbytes: int):
-        self.__cuda_array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False),
-                                         "version": 2, "strides": None}
-
-
-def _copy_device_bytes(ptr: int, nbytes: int, dtype=torch.uint8, pad_to: int = 1) -> torch.Tensor:
-    dev = torch.device("cuda", torch.cuda.current_device())
-    out = torch.zeros(max(pad_to, nbytes), dtype=torch.uint8, device=dev)
-    if nbytes > 0:
-        out[:nbytes].copy_(torch.as_tensor(_DeviceBytes(ptr, nbytes), device=dev))
-    return out.view(dtype) if dtype != torch.uint8 else out
-
-
 class BatchedGroupBy:
     """A plan over ``instances``: a list of ``(key_column, [values_column per
     request])``; ``aggregations[r]`` is the aggregation list of request r."""
@@ -115,31 +98,32 @@ class BatchedGroupBy:
     def num_groups(self, i: int) -> int:
         return int(_lib.lib().mig_batch_num_groups(self._handle, i))
 
-    @staticmethod
-    def _copy(out: _lib.OutColumn) -> Column:
-        data = _copy_device_bytes(out.data, out.size * width(TypeId(out.type_id)))
-        mask = None
-        if out.null_mask:
-            words = (out.size + 31) // 32
-            mask = _copy_device_bytes(out.null_mask, words * 4, torch.int32, pad_to=4)
-        return Column(out.type_id, out.size, data, mask, out.null_count)
-
     def result(self, i: int) -> Tuple[Table, List[Table]]:
         """Instance ``i``'s unique keys and per-request results, copied out of
         the plan's buffers on torch's current stream (valid after
         ``synchronize``, on the stream the plan ran on or one ordered after it)."""
         L = _lib.lib()
-        out = _lib.OutColumn()
-        _lib.check(L.mig_batch_result_key(self._handle, i, ctypes.byref(out)))
-        keys = self._copy(out)
-        results = []
-        for r, al in enumerate(self._aggs):
-            cols = []
-            for a in range(len(al)):
-                _lib.check(L.mig_batch_result_column(self._handle, i, r, a, ctypes.byref(out)))
-                cols.append(self._copy(out))
-            results.append(Table(cols))
-        return Table([keys]), results
+        n = 1 + sum(len(al) for al in self._aggs)
+        cols = (_lib.OutColumn * n)()
+        data_at, mask_at = (ctypes.c_int64 * n)(), (ctypes.c_int64 * n)()
+        total = ctypes.c_int64()
+        _lib.check(L.mig_batch_result(self._handle, i, cols, data_at, mask_at, ctypes.byref(total)))
+        # the columns share one buffer, filled by one copy
+        dev = torch.device("cuda", torch.cuda.current_device())
+        make = torch.empty if cols[0].size else torch.zeros
+        buf = make(total.value, dtype=torch.uint8, device=dev)
+        _lib.check(L.mig_batch_result_copy(self._handle, i, ctypes.c_void_p(buf.data_ptr()), _stream_handle(None)))
+        out = []
+        for c, at, mat in zip(cols, data_at, mask_at):
+            size, tid = c.size, TypeId(c.type_id)
+            data = buf[at:at + max(1, size * width(tid))]
+            mask = buf[mat:mat + max(4, (size + 31) // 32 * 4)].view(torch.int32) if mat >= 0 else None
+            out.append(Column(tid, size, data, mask, c.null_count))
+        results, k = [], 1
+        for al in self._aggs:
+            results.append(Table(out[k:k + len(al)]))
+            k += len(al)
+        return Table(out[:1]), results
 
     def close(self) -> None:
         if self._handle:

@@ -749,6 +749,54 @@ mig_column batch_result_column(mig_batch_plan const* plan, int32_t instance, int
   return c;
 }
 
+int64_t batch_result(mig_batch_plan const* plan, int32_t instance, mig_column* out, int64_t* data_at,
+                     int64_t* mask_at)
+{
+  out[0] = batch_result_key(plan, instance);
+  int c  = 1;
+  for (int32_t r = 0; r < plan->num_requests; r++)
+    for (int32_t a = 0; a < plan->agg_begin[size_t(r) + 1] - plan->agg_begin[size_t(r)]; a++)
+      out[c++] = batch_result_column(plan, instance, r, a);
+  int64_t total = 0;
+  auto place    = [&](int64_t bytes) {
+    int64_t const at = total;
+    total += std::max<int64_t>(256, (bytes + 255) & ~int64_t(255));
+    return at;
+  };
+  for (int k = 0; k < c; k++) {
+    data_at[k] = place(int64_t(out[k].size) * type_width(out[k].type_id));
+    mask_at[k] = out[k].null_mask ? place((int64_t(out[k].size) + 31) / 32 * 4) : -1;
+  }
+  return total;
+}
+
+void batch_result_copy(mig_batch_plan const* plan, int32_t instance, void* dst, hipStream_t stream)
+{
+  MIG_EXPECTS(plan != nullptr, "null batch plan");
+  size_t const n = 1 + size_t(plan->agg_begin[size_t(plan->num_requests)]);
+  std::vector<mig_column> cols(n);
+  std::vector<int64_t> data_at(n), mask_at(n);
+  (void)batch_result(plan, instance, cols.data(), data_at.data(), mask_at.data());
+  copy_segments L{};
+  auto flush = [&] {
+    launch_copy_segments(L, static_cast<uint8_t*>(dst), stream);
+    L.n = 0;
+  };
+  auto add = [&](void const* src, int64_t at, int64_t bytes) {
+    if (bytes <= 0) return;
+    if (L.n == MAX_COPY_SEGMENTS) flush();
+    L.src[L.n]     = static_cast<uint8_t const*>(src);
+    L.at[L.n]      = at;
+    L.bytes[L.n++] = bytes;
+  };
+  for (size_t k = 0; k < n; k++) {
+    add(cols[k].data, data_at[k], int64_t(cols[k].size) * type_width(cols[k].type_id));
+    if (mask_at[k] >= 0) add(cols[k].null_mask, mask_at[k], (int64_t(cols[k].size) + 31) / 32 * 4);
+  }
+  flush();
+  MIG_HIP_TRY(hipGetLastError());
+}
+
 void batch_plan_free(mig_batch_plan* plan) { delete plan; }
 
 }  // namespace mig

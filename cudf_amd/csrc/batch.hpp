@@ -76,6 +76,15 @@ struct batch_params {
   int32_t lds_bytes;
 };
 
+// Device ranges (8-byte aligned) copied to byte offsets (8-byte aligned) of one buffer.
+constexpr int MAX_COPY_SEGMENTS = 64;
+struct copy_segments {
+  int32_t n;
+  uint8_t const* src[MAX_COPY_SEGMENTS];
+  int64_t at[MAX_COPY_SEGMENTS];
+  int64_t bytes[MAX_COPY_SEGMENTS];
+};
+void launch_copy_segments(copy_segments const& L, uint8_t* dst, hipStream_t s);
 void launch_batch_sample(batch_params const* dB, int32_t n_inst, int32_t per_inst, uint64_t* tables,
                          uint32_t table_slots, uint32_t* counters, hipStream_t s);
 void launch_batch_init(batch_params const* dB, batch_params const& hB, int num_cus, hipStream_t s);

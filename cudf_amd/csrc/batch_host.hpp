@@ -16,6 +16,9 @@ int32_t batch_num_groups(mig_batch_plan const* plan, int32_t instance);
 mig_column batch_result_key(mig_batch_plan const* plan, int32_t instance);
 mig_column batch_result_column(mig_batch_plan const* plan, int32_t instance, int32_t request,
                                int32_t agg);
+int64_t batch_result(mig_batch_plan const* plan, int32_t instance, mig_column* out, int64_t* data_at,
+                     int64_t* mask_at);
+void batch_result_copy(mig_batch_plan const* plan, int32_t instance, void* dst, hipStream_t stream);
 void batch_plan_free(mig_batch_plan* plan);
 
 }  // namespace mig

@@ -794,6 +794,30 @@ void launch_batch_valid_counts(batch_params const* dB, batch_params const& hB, h
   hipLaunchKernelGGL(k_batch_valid_counts, dim3(hB.n_inst, hB.num_outs + 1), dim3(BBLOCK), 0, s, dB);
 }
 
+// One launch for all of an instance's columns (a copy each, and a fill of each
+// destination, made 224 launches of 2.4 us for 16 instances of 7 columns).
+__global__ void __launch_bounds__(BBLOCK) k_copy_segments(copy_segments L, uint8_t* dst)
+{
+  int const i         = blockIdx.y;
+  auto const src      = gp(L.src[i]);
+  auto const out      = gp(dst + L.at[i]);
+  int64_t const words = L.bytes[i] / 8;
+  int64_t const t0    = int64_t(blockIdx.x) * BBLOCK + threadIdx.x;
+  for (int64_t k = t0; k < words; k += int64_t(gridDim.x) * BBLOCK)
+    reinterpret_cast<gmem<uint64_t>*>(out)[k] = reinterpret_cast<gmem<uint64_t const>*>(src)[k];
+  int64_t const tail = words * 8 + t0;
+  if (tail < L.bytes[i]) out[tail] = src[tail];
+}
+
+void launch_copy_segments(copy_segments const& L, uint8_t* dst, hipStream_t s)
+{
+  if (L.n == 0) return;
+  int64_t most = 0;
+  for (int i = 0; i < L.n; i++) most = std::max(most, L.bytes[i]);
+  int64_t const blocks = std::max<int64_t>(1, std::min<int64_t>(64, (most / 8 + 4 * BBLOCK - 1) / (4 * BBLOCK)));
+  hipLaunchKernelGGL(k_copy_segments, dim3(blocks, L.n), dim3(BBLOCK), 0, s, L, dst);
+}
+
 void prepare_batch_aggregate(int32_t lds_bytes)
 {
   allow_dynamic_lds(reinterpret_cast<void const*>(&k_batch_aggregate<256>), lds_bytes);

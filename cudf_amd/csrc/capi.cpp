@@ -269,6 +269,23 @@ mig_status mig_batch_result_column(const mig_batch_plan* plan, int32_t instance,
   });
 }
 
+mig_status mig_batch_result(const mig_batch_plan* plan, int32_t instance, mig_column* out, int64_t* data_at,
+                            int64_t* mask_at, int64_t* total_bytes)
+{
+  return guarded([&] {
+    if (!out || !data_at || !mask_at || !total_bytes) mig::fail(MIG_ERROR_LOGIC, "null output array");
+    *total_bytes = mig::batch_result(plan, instance, out, data_at, mask_at);
+  });
+}
+
+mig_status mig_batch_result_copy(const mig_batch_plan* plan, int32_t instance, void* dst, void* stream)
+{
+  return guarded([&] {
+    if (!dst) mig::fail(MIG_ERROR_LOGIC, "null destination");
+    mig::batch_result_copy(plan, instance, dst, static_cast<hipStream_t>(stream));
+  });
+}
+
 void mig_batch_plan_free(mig_batch_plan* plan) { mig::batch_plan_free(plan); }
 
 int32_t mig_table_num_rows(const mig_table* t) { return t ? t->num_rows : 0; }

@@ -246,6 +246,14 @@ int32_t mig_batch_num_groups(const mig_batch_plan* plan, int32_t instance);
 mig_status mig_batch_result_key(const mig_batch_plan* plan, int32_t instance, mig_column* out);
 mig_status mig_batch_result_column(const mig_batch_plan* plan, int32_t instance, int32_t request,
                                    int32_t agg, mig_column* out);
+/* An instance's key column (out[0]) and its result columns in request order,
+ * and where mig_batch_result_copy puts their parts: data_at[c] and mask_at[c]
+ * (-1: no mask) are byte offsets, multiples of 256, into a buffer of
+ * *total_bytes.  The arrays hold 1 + (all aggregations) entries. */
+mig_status mig_batch_result(const mig_batch_plan* plan, int32_t instance, mig_column* out, int64_t* data_at,
+                            int64_t* mask_at, int64_t* total_bytes);
+/* Copies those columns into `dst` (device memory) on `stream`. */
+mig_status mig_batch_result_copy(const mig_batch_plan* plan, int32_t instance, void* dst, void* stream);
 void mig_batch_plan_free(mig_batch_plan* plan);
 
 /* ---- library -------------------------------------------------------------- */
