@@ -104,7 +104,7 @@ constexpr int32_t BATCH_SAMPLE = 4096;  // sampled rows per instance
 // per-row device-wide atomics the batched kernels fall back to when an
 // instance's groups exceed what LDS pre-aggregation takes.
 constexpr int32_t BATCH_SOLO_ROWS   = 1 << 20;
-constexpr double BATCH_SOLO_GROUPS  = 65536.0;
+constexpr double BATCH_SOLO_GROUPS  = 8192.0;  // what BATCH_MAX_PARTS LDS parts hold
 
 int32_t default_i(int32_t v, int32_t d) { return v == 0 ? d : v; }
 

@@ -702,8 +702,11 @@ class groupby_call {
   int64_t aggregate_partitioned();
   int64_t aggregate_hot_split();
   bool partitionable();
+  bool partitioning_pays();
+  bool few_groups();
   int64_t aggregate_global();
   int32_t lds_most_slots();
+  int32_t direct_slots();
   void lds_layout(int32_t slots);
   size_t alloc_table(uint64_t cap);
   void alloc_dump(int64_t blocks);
@@ -1319,6 +1322,27 @@ bool groupby_call::partitionable()
   return rpa_ok;
 }
 
+// Whether the partitioned path beats the table paths.  The device-wide table
+// runs at 24 G atomics/s whatever its size (7 G/s on a thousand addresses), the
+// partitioned path at a few passes over the rows plus some 40 us of launches.
+// Measured, us a call, table / partitioned: one fixed-width key, one sum
+// 120K rows 148 / 152, 240K 160 / 157, 1M 213 / 183, 16M 1,022 / 567; four
+// accumulators 60K 158 / 160, 240K 205 / 170, 4M 861 / 262, 16M 2,962 / 613
+// (5,000 to N / 3 groups alike).  Few groups take the LDS tables instead.
+// General keys (hashing and verifying rows costs more): five accumulators
+// 100K 280 / 310, 300K 355 / 325, 6M 1,847 / 995; one accumulator no gain
+// (300K 282 / 291, 6M 846 / 895) but with few groups (600: 300K 376 / 292, 6M
+// 2,069 / 994).  A key on many rows would make a straggler of its bin.
+bool groupby_call::partitioning_pays()
+{
+  gb_params const& p  = P();
+  int const atomics   = nf_ + (p.need_count_all ? 1 : 0);
+  if (p.key_mode == KM_INLINE) return N >= 200'000 && !few_groups() && !heavy_hitters();
+  if (N >= (1 << 20) && est_ >= 65536) return !heavy_hitters();
+  bool const straggler = sampled_ > 0.0 && double(max_mult_) * 64.0 >= sampled_;
+  return N >= 300'000 && (atomics >= 3 || est_ <= 1024.0) && !straggler;
+}
+
 // Radix-partitioned LDS aggregation for high cardinality: returns the number
 // of groups, or -1 when the path does not apply (or its bins overflowed three
 // times) and the device-wide table takes the call.
@@ -1350,8 +1374,7 @@ int64_t groupby_call::aggregate_partitioned()
   bool use_rpa = false;
   if (forced == MIG_STRATEGY_PARTITIONED || forced == MIG_STRATEGY_PARTITIONED_EXACT) use_rpa = rpa_ok;
   else if (forced == MIG_STRATEGY_AUTO)  // and the estimate fits the largest partition
-    use_rpa = rpa_ok && (split_ || (N >= (1 << 20) && est_ >= 65536 && !heavy_hitters())) &&
-              est_ <= double(int64_t(1) << RPA_MAX_LOG_BINS) * max_fill;
+    use_rpa = rpa_ok && (split_ || partitioning_pays()) && est_ <= double(int64_t(1) << RPA_MAX_LOG_BINS) * max_fill;
   if (!use_rpa) return -1;
   int64_t const rows = p.num_rows;  // the input's, or those left after aggregate_hot_split
 
@@ -1448,6 +1471,8 @@ int64_t groupby_call::aggregate_partitioned()
   double const per_bin = 0.66 * double(S_slots);
   int log_bins = 1;
   while (log_bins < RPA_MAX_LOG_BINS && double(int64_t(1) << log_bins) * per_bin < est_) log_bins++;
+  // a bin is one workgroup's: at least 256 of them while that leaves each 4,096 rows
+  while (log_bins < RPA_MAX_LOG_FANOUT && (rows >> log_bins) > 4096) log_bins++;
   // the last doubling only for estimates that would fill 2^15 bins past
   // 0.78·S (measured: 2^15 fuller bins beat 2^16 half-empty ones by ~0.8 ms
   // at 25M groups)
@@ -1625,13 +1650,35 @@ int64_t groupby_call::aggregate_partitioned()
 // Most slots of an LDS partial table (and of the variance pass's).
 int32_t groupby_call::lds_most_slots()
 {
-  int32_t row_bytes = 8, m2_bytes = 8;
+  int32_t row_bytes = 8, m2_bytes = 12;
   for (int f = 0; f < nf_; f++) {
-    if (P().fields[f].kind == FK_M2) m2_bytes += 8;
+    if (P().fields[f].kind == FK_M2) m2_bytes += 16;
     else row_bytes += rpa_lds_width(P().fields[f].kind, true);  // float32 sums in float64
   }
   if (P().need_count_all) row_bytes += 4;
   return (LDS_PREAGG_BUDGET / std::max(row_bytes, m2_bytes) - LDS_EXTRA_SLOTS - 16) & ~63;
+}
+
+// Whether the LDS partial tables hold the (estimated) groups of a fixed-width
+// key: at least 1.45x the estimate's slots, or a slot for every key of the
+// sampled range.
+bool groupby_call::few_groups()
+{
+  if (P().key_mode != KM_INLINE || any_arg_ || nf_ > 64) return false;
+  double const most = double(lds_most_slots());
+  return direct_slots() > 0 ||
+         (est_ <= double(LDS_PREAGG_MAX_GROUPS) && std::max(256.0, 1.45 * est_ + 64.0) <= most);
+}
+
+// Slots of LDS tables indexed by an integer key's value: the sampled range,
+// when it fits and does not hold the tables' empty marker; else 0.
+int32_t groupby_call::direct_slots()
+{
+  if (key_min_ > key_max_) return 0;
+  uint64_t const span = uint64_t(key_max_) - uint64_t(key_min_);
+  int32_t const most  = lds_most_slots();
+  if (most <= 0 || span >= uint64_t(most) || EMPTY_KEY - uint64_t(key_min_) <= span + 64) return 0;
+  return int32_t((span + 64) & ~uint64_t(63));
 }
 
 // Lays out LDS partial tables of `slots` slots (lds_bytes stays 0 when they
@@ -1639,27 +1686,30 @@ int32_t groupby_call::lds_most_slots()
 void groupby_call::lds_layout(int32_t slots)
 {
   gb_params& p = P();
-  int32_t off = (slots + LDS_EXTRA_SLOTS) * 8, m2_off = off;
+  int32_t off = (slots + LDS_EXTRA_SLOTS) * 8;
   for (int f = 0; f < nf_; f++) {
     field_desc& F = p.fields[f];
-    if (F.kind == FK_M2) {
-      p.lds_m2_off[f] = m2_off;
-      m2_off += slots * 8;
-    } else {
-      F.lds_off = off;
-      off += ((slots + LDS_EXTRA_SLOTS) * rpa_lds_width(F.kind, true) + 7) & ~7;
-    }
+    if (F.kind == FK_M2) continue;
+    F.lds_off = off;
+    off += ((slots + LDS_EXTRA_SLOTS) * rpa_lds_width(F.kind, true) + 7) & ~7;
   }
   p.lds_count_off = -1;
   if (p.need_count_all) {
     p.lds_count_off = off;
     off += ((slots + LDS_EXTRA_SLOTS) * 4 + 7) & ~7;
   }
-  int32_t const bytes = std::max(off, m2_off);
-  if (bytes > LDS_PREAGG_BUDGET || nf_ > 64) return;
-  p.lds_slots = slots;
-  p.lds_fill  = slots * 17 / 20;
-  p.lds_bytes = bytes;
+  // the variance pass: keys, device-wide slots, mean and deviations per field
+  int32_t m2_off = (slots + LDS_EXTRA_SLOTS) * 12;
+  for (int f = 0; f < nf_; f++) {
+    if (p.fields[f].kind != FK_M2) continue;
+    p.lds_m2_off[f] = (m2_off + 7) & ~7;
+    m2_off          = p.lds_m2_off[f] + (slots + LDS_EXTRA_SLOTS) * 16;
+  }
+  if (std::max(off, m2_off) > LDS_PREAGG_BUDGET || nf_ > 64) return;
+  p.lds_slots    = slots;
+  p.lds_fill     = slots * 17 / 20;
+  p.lds_bytes    = off;
+  p.lds_m2_bytes = m2_off;
 }
 
 // The device-wide table of `cap` slots and its accumulators; returns their bytes.
@@ -1708,7 +1758,7 @@ int64_t groupby_call::aggregate_hot_split()
 {
   gb_params& p = P();
   if (mem_ || g_strategy.load() != MIG_STRATEGY_AUTO || p.key_mode != KM_INLINE || any_arg_ || !heavy_hitters() ||
-      N < (1 << 20) || est_ <= double(LDS_PREAGG_MAX_GROUPS) || sample_table_ == nullptr || !partitionable())
+      N < (1 << 20) || few_groups() || sample_table_ == nullptr || !partitionable())
     return -1;
   int32_t const slots = lds_most_slots();
   if (slots < 1024) return -1;
@@ -1817,27 +1867,22 @@ int64_t groupby_call::aggregate_global()
   p.lds_bytes        = 0;
   // workgroup-local tables for few groups, or for hot keys among many
   // groups (rows of keys that find no room go to the device-wide table)
-  if (p.key_mode == KM_INLINE && !any_arg_ && (est_ <= double(LDS_PREAGG_MAX_GROUPS) || heavy_hitters()) &&
-      forced != MIG_STRATEGY_PARTITIONED) {
+  if (p.key_mode == KM_INLINE && !any_arg_ && forced != MIG_STRATEGY_PARTITIONED) {
     // A third of the slots filled (the longest probe of a wave's 64 rows is
-    // what it waits for), or as many as fit: 1.2x the estimate at 85% filled
-    // is the least.  Hot keys among many groups: as many slots as fit.
-    int32_t const most  = lds_most_slots();
-    double const least  = std::max(256.0, 1.45 * est_ + 64.0);
-    bool const few      = est_ <= double(LDS_PREAGG_MAX_GROUPS) && least <= double(most);
-    bool hot            = !few && heavy_hitters() && most >= 1024;
-    int32_t S_l         = most;
+    // what it waits for), or as many as fit.  Integer keys of a range that fits
+    // (ids, dictionary codes): a slot per key of the sampled range, found
+    // without probing.  Hot keys among many groups: as many slots as fit.
+    int32_t const most = lds_most_slots();
+    bool const few     = few_groups();
+    bool const hot     = !few && heavy_hitters() && most >= 1024;
+    int32_t S_l        = most;
     if (few) S_l = std::min<int32_t>(most, std::max<int32_t>(256, (int32_t(3.0 * est_) + 63) & ~63));
-    // Integer keys of a range that fits (ids, dictionary codes): a slot per
-    // key of the sampled range, found without probing.
-    uint64_t const span = key_min_ <= key_max_ ? uint64_t(key_max_) - uint64_t(key_min_) : UINT64_MAX;
-    p.lds_direct        = span < uint64_t(most) && EMPTY_KEY - uint64_t(key_min_) > span + 64;
-    p.lds_key_min       = key_min_;
-    if (p.lds_direct) {
-      S_l = int32_t((span + 64) & ~uint64_t(63));
-      hot = false;
-    }
-    if (few || hot || p.lds_direct) lds_layout(S_l);
+    int32_t const direct = direct_slots();
+    p.lds_direct         = direct > 0;
+    p.lds_key_min        = key_min_;
+    if (direct > 0) S_l = direct;
+    p.lds_hot = hot;
+    if (few || hot) lds_layout(S_l);
     if (p.lds_bytes > 0) {
       // one workgroup per CU (16 waves): more would only add tables to merge
       // enough rows per group and workgroup that its table pays off (hot keys:

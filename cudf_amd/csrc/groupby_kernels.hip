@@ -626,8 +626,7 @@ void launch_second_pass(gb_params const* dP, gb_params const& hP, int num_cus, h
 // Few groups (one fixed-width key): per-workgroup partial tables in LDS, merged
 // once per workgroup.  A global atomic per row and field would run at 24 G/s on
 // this device (7 G/s on a thousand addresses); LDS atomics take 5-12 ns per
-// wave and CU.  Rows whose key finds no room go to the device-wide table.  The
-// variance pass keys an LDS table by group slot.
+// wave and CU.  Rows whose key finds no room go to the device-wide table.
 //
 // Bound by instruction issue and LDS operations, so: descriptors come from the
 // lanes of a register (lds_plan); rows that don't count go to a spare slot of
@@ -1256,7 +1255,173 @@ __global__ void __launch_bounds__(LBLOCK) k_merge_lds(gb_params const* __restric
   }
 }
 
+// The variance pass over the groups of the finished device-wide table: their
+// means are loaded into LDS once, so a row costs its probe (or none: DIRECT, as
+// in k_aggregate_lds), one read and one add per column.  Rows whose group found
+// no room update the device-wide table.  Accumulators: mean, then Σ(x - mean)²,
+// per FK_M2 field at lds_m2_off.
+template <bool DIRECT>
 __global__ void __launch_bounds__(LBLOCK) k_second_pass_lds(gb_params const* __restrict__ Pp)
+{
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  __shared__ uint32_t fill_sh;
+  gb_params const& P  = *Pp;
+  int const S         = P.lds_slots;
+  int const NS        = S + LDS_EXTRA_SLOTS;
+  lds_plan const A    = load_lds_plan(P);
+  int const nfields   = P.num_fields;
+  int const lane      = int(threadIdx.x & 63u);
+  uint32_t const m2_l = uint32_t(P.lds_m2_off[lane < nfields ? lane : 0]);
+  auto* tkeys         = reinterpret_cast<uint64_t*>(lds);
+  auto* tslots        = reinterpret_cast<uint32_t*>(tkeys + NS);  // device-wide slots
+  auto mean           = [&](int32_t off, int i) { return reinterpret_cast<double*>(lds + off) + i; };
+  auto m2             = [&](int32_t off, int i) { return reinterpret_cast<double*>(lds + off) + NS + i; };
+  for (int i = threadIdx.x; i < NS; i += LBLOCK) {
+    tkeys[i]  = EMPTY_KEY;
+    tslots[i] = 0xffffffffu;
+  }
+  for (int f = 0; f < nfields; f++) {
+    if ((lane_value(A.fd, f) & 0xffu) != FK_M2) continue;
+    int32_t const off = int32_t(lane_value(m2_l, f));
+    for (int i = threadIdx.x; i < 2 * NS; i += LBLOCK) *mean(off, i) = 0.0;
+  }
+  if (threadIdx.x == 0) fill_sh = 0;
+  __syncthreads();
+  dcol const kc         = P.keys[0];
+  int32_t const kst     = kc.storage;
+  int64_t const key_min = P.lds_key_min;
+  for (int64_t g = threadIdx.x; g < int64_t(P.cap) + 2; g += LBLOCK) {
+    int id = -1;
+    if (g < int64_t(P.cap)) {
+      uint64_t c[1] = {gp(P.slot_keys)[g]};
+      if (c[0] == EMPTY_KEY) continue;
+      if constexpr (DIRECT) {
+        canon_rows(kst, c);
+        uint64_t const i = c[0] - uint64_t(key_min);
+        if (i < uint64_t(S)) id = int(i);
+      } else {
+        id = lds_insert_any(tkeys, &fill_sh, c[0], lds_key_hash(c[0]), EMPTY_KEY, S, uint32_t(P.lds_fill));
+      }
+    } else if (P.special[g - int64_t(P.cap)]) {
+      id = S + int(g - int64_t(P.cap));
+    }
+    if (id < 0) continue;
+    tslots[id] = uint32_t(g);  // the table of few groups is small
+    for (int f = 0; f < nfields; f++) {
+      field_desc const& F = P.fields[f];
+      if (F.kind == FK_M2)
+        *mean(P.lds_m2_off[f], id) = field_as_double(P.fields[F.aux_sum], g) / double(count_of(P, F.aux_count, g));
+    }
+  }
+  __syncthreads();
+  int const kw          = storage_width(kst);
+  bool const skip_nulls = P.skip_null_keys != 0;
+  auto const kdata      = gp(kc.data);
+  auto const kmask      = gp(kc.mask);
+  uint32_t const koff   = uint32_t(kc.mask_offset);
+  uint32_t const n      = uint32_t(P.num_rows);
+  constexpr int U       = LDS_ROWS;
+  int const spare       = S + 2 + lane;
+  uint32_t const stride = gridDim.x * (LBLOCK * U);
+  for (uint32_t w0 = blockIdx.x * (LBLOCK * U); w0 < n; w0 += stride) {
+    uint32_t const r0 = w0 + threadIdx.x;
+    uint64_t key[U];
+    uint32_t kwv[U];
+    if (kmask) load_valid_words(kmask, koff, r0, n, kwv);
+    load_chunk<LBLOCK>(kdata, kw, r0, n, key);
+    int id[U];
+    uint32_t full = 0, probe = 0, h[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      id[u]           = spare;
+      bool const in   = r0 + uint32_t(u) * LBLOCK < n;
+      bool const null = kmask && !((kwv[u] >> ((r0 + koff) & 31u)) & 1u);
+      if (in && null && !skip_nulls) id[u] = S + 1;
+      if (kst == ST_F32) key[u] = normalize_f32_bits(uint32_t(key[u]));
+      else if (kst == ST_F64) key[u] = normalize_f64_bits(key[u]);
+      else if (kst == ST_BOOL) key[u] = key[u] != 0;
+      if (in && !null && key[u] == EMPTY_KEY) id[u] = S;
+      h[u] = lds_key_hash(key[u]);
+      probe |= uint32_t(in && !null && key[u] != EMPTY_KEY) << u;
+    }
+    int found[U];
+    if constexpr (DIRECT) {
+      uint64_t c[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) c[u] = key[u];
+      canon_rows(kst, c);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        uint64_t const i = c[u] - uint64_t(key_min);
+        found[u]         = i < uint64_t(S) ? int(i) : -1;
+      }
+    } else {
+      lds_insert_rows(tkeys, &fill_sh, key, h, probe, S, 0u, found);  // finds only
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      bool const mine = (probe >> u) & 1u;
+      if (mine && found[u] >= 0) id[u] = found[u];
+      full |= uint32_t(mine && found[u] < 0) << u;
+    }
+    for (int i = 0; i < A.ncols; i++) {
+      uint32_t const cd = lane_value(A.cd, i);
+      int const fb = int((cd >> 8) & 0xffu), fe = int((cd >> 16) & 0xffu), st = int(cd & 0x7fu);
+      int m2f = -1;
+      for (int f = fb; f < fe; f++)
+        if ((lane_value(A.fd, f) & 0xffu) == FK_M2) m2f = f;
+      if (m2f < 0) continue;
+      int32_t const off = int32_t(lane_value(m2_l, m2f));
+      lds_column col;
+      load_lds_column(A, i, r0, n, col);
+      canon_rows(st, col.c);
+      int at[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) at[u] = id[u];
+      if (cd & 0x80u) {
+        uint32_t const sh = (r0 + lane_value(A.mask_offset, i)) & 31u;
+#pragma unroll
+        for (int u = 0; u < U; u++) at[u] = (col.w[u] >> sh) & 1u ? at[u] : spare;
+      }
+      double mu[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) mu[u] = *mean(off, at[u]);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        double const d = canon_double(st, col.c[u]) - mu[u];
+        __hip_atomic_fetch_add(m2(off, at[u]), d * d, __ATOMIC_RELAXED, WG_SCOPE);
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(full != 0) == 0) continue;
+    for (int u = 0; u < U; u++) {  // groups without room in LDS
+      if (!((full >> u) & 1u)) continue;
+      int64_t const row  = int64_t(r0 + uint32_t(u) * LBLOCK);
+      int64_t const slot = locate<KM_INLINE, false>(P, row);
+      if (slot < 0) continue;
+      for (int f = 0; f < nfields; f++) {
+        field_desc const& F = P.fields[f];
+        if (F.kind != FK_M2 || !dcol_valid(P.vals[F.vcol], row)) continue;
+        double const mu = field_as_double(P.fields[F.aux_sum], slot) / double(count_of(P, F.aux_count, slot));
+        double const d  = load_value(P.vals[F.vcol], row).d - mu;
+        gadd_f64(reinterpret_cast<double*>(field_at(F, slot)), d * d);
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < S + 2; i += LBLOCK) {
+    uint32_t const slot = tslots[i];
+    if (slot == 0xffffffffu) continue;
+    for (int f = 0; f < nfields; f++) {
+      if (P.fields[f].kind != FK_M2) continue;
+      double const part = *m2(P.lds_m2_off[f], i);
+      if (part != 0.0) gadd_f64(reinterpret_cast<double*>(field_at(P.fields[f], int64_t(slot))), part);
+    }
+  }
+}
+
+// The same for hot keys among many groups: a table of group slots filled as the
+// rows come, so that it holds the hot ones.
+__global__ void __launch_bounds__(LBLOCK) k_second_pass_hot(gb_params const* __restrict__ Pp)
 {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ uint32_t fill_sh;
@@ -1266,9 +1431,11 @@ __global__ void __launch_bounds__(LBLOCK) k_second_pass_lds(gb_params const* __r
   int const S        = P.lds_slots;
   auto* tslots       = reinterpret_cast<uint64_t*>(lds);
   for (int i = threadIdx.x; i < S; i += LBLOCK) tslots[i] = NO;
+  // partials of M2 field f
+  auto m2 = [&](int f, int i) { return lds_at<double>(lds, P.lds_m2_off[f], i); };
   for (int f = 0; f < P.num_fields; f++) {
     if (P.fields[f].kind != FK_M2) continue;
-    for (int i = threadIdx.x; i < S; i += LBLOCK) *lds_at<double>(lds, P.lds_m2_off[f], i) = 0.0;
+    for (int i = threadIdx.x; i < S; i += LBLOCK) *m2(f, i) = 0.0;
   }
   if (threadIdx.x == 0) fill_sh = 0;
   __syncthreads();
@@ -1296,7 +1463,7 @@ __global__ void __launch_bounds__(LBLOCK) k_second_pass_lds(gb_params const* __r
         double const cnt  = double(count_of(P, F.aux_count, slot));
         double const mean = field_as_double(P.fields[F.aux_sum], slot) / cnt;
         double const d    = v.d - mean;
-        if (id >= 0) __hip_atomic_fetch_add(lds_at<double>(lds, P.lds_m2_off[f], id), d * d, __ATOMIC_RELAXED, WG);
+        if (id >= 0) __hip_atomic_fetch_add(m2(f, id), d * d, __ATOMIC_RELAXED, WG);
         else gadd_f64(reinterpret_cast<double*>(field_at(F, slot)), d * d);
       }
     }
@@ -1307,7 +1474,7 @@ __global__ void __launch_bounds__(LBLOCK) k_second_pass_lds(gb_params const* __r
     if (slot == NO) continue;
     for (int f = 0; f < P.num_fields; f++) {
       if (P.fields[f].kind != FK_M2) continue;
-      double const part = *lds_at<double>(lds, P.lds_m2_off[f], i);
+      double const part = *m2(f, i);
       if (part != 0.0) gadd_f64(reinterpret_cast<double*>(field_at(P.fields[f], int64_t(slot))), part);
     }
   }
@@ -1350,8 +1517,13 @@ void launch_aggregate_lds(gb_params const* dP, gb_params const& hP, int64_t bloc
 void launch_second_pass_lds(gb_params const* dP, gb_params const& hP, int64_t blocks, hipStream_t s)
 {
   if (hP.num_rows <= 0) return;
-  allow_dynamic_lds(reinterpret_cast<void const*>(&k_second_pass_lds), hP.lds_bytes);
-  hipLaunchKernelGGL(k_second_pass_lds, dim3(blocks), dim3(LBLOCK), hP.lds_bytes, s, dP);
+  auto run = [&](auto* kernel) {
+    allow_dynamic_lds(reinterpret_cast<void const*>(kernel), hP.lds_m2_bytes);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(LBLOCK), hP.lds_m2_bytes, s, dP);
+  };
+  if (hP.lds_hot) run(&k_second_pass_hot);
+  else if (hP.lds_direct) run(&k_second_pass_lds<true>);
+  else run(&k_second_pass_lds<false>);
 }
 
 // ---------------------------------------------------------------------------

@@ -174,12 +174,14 @@ struct gb_params {
   // fields[f].lds_off (lds_slots + LDS_EXTRA_SLOTS elements of the field's
   // width; slots lds_slots and lds_slots + 1 hold the EMPTY_KEY and null-key
   // groups, then one slot per lane takes the rows that do not count) and
-  // the row counts at lds_count_off (-1: none); the variance pass reuses the
-  // bytes for a table of group slots and the M2 partials at lds_m2_off[f]
+  // the row counts at lds_count_off (-1: none); the variance pass has the same
+  // slots, with the means and then the M2 partials at lds_m2_off[f]
   int32_t lds_slots;
   int32_t lds_fill;
   int32_t lds_count_off;
   int32_t lds_bytes;
+  int32_t lds_m2_bytes;
+  int32_t lds_hot;  // hot keys among many groups: the tables hold the keys that came first
   int32_t lds_m2_off[MAX_FIELDS];
   // many workgroups: each stores its table here (lds_dump_stride bytes apart,
   // the last 8 telling which special groups it has) instead of merging it

@@ -86,3 +86,36 @@ def test_hot_keys_apart_from_the_rest(key_dtype, policy, nulls):
     i = host_col(rng.integers(0, 10_000, n).astype(np.int32), rng.random(n) >= 0.03)
     assert_parity([key], [(f, C2_AGGS), (i, C2_AGGS)], policy)
     assert _stats()["lds_preagg"] == 1.0 and _stats()["strategy"] == 1
+
+
+@pytest.mark.parametrize("n,card,general", [(199_999, 9_000, False), (200_000, 9_000, False), (600_001, 5_000, False),
+                                            (1_100_003, 20_000, False), (299_999, 3_000, True), (300_000, 3_000, True)])
+def test_path_for_the_rows_and_groups(n, card, general):
+    """Both sides of the line between the device-wide table and the
+    partitioned path (with few groups its bins are many and nearly empty)."""
+    rng = np.random.default_rng(n)
+    k = rng.integers(-2**40, 2**40, card)[rng.integers(0, card, n)]
+    keys = [host_col(k, rng.random(n) >= 0.01)]
+    if general:
+        keys.append(host_col((k % 7).astype(np.int16)))
+    v = host_col(rng.standard_normal(n), rng.random(n) >= 0.04)
+    i = host_col(rng.integers(-9, 9, n).astype(np.int8))
+    assert_parity(keys, [(v, C2_AGGS), (i, [(AGG["SUM"], 1), (AGG["MAX"], 1)])])
+    assert _stats()["strategy"] == (2 if n >= (300_000 if general else 200_000) else 1)
+
+
+@pytest.mark.parametrize("card", [1, 20, 700, 3_000])
+@pytest.mark.parametrize("spread", [1, 1_000_003])
+def test_variance_of_few_groups(card, spread):
+    """The variance pass with the means in LDS, slots by value and by probe;
+    null keys as a group; NaN, infinities and groups of one value."""
+    rng = np.random.default_rng(card + spread)
+    n = 90_001
+    k = rng.integers(0, card, n) * spread
+    k[:3] = [10**15, 10**15 + 1, -10**15]
+    x = rng.standard_normal(n) * 1e3 + 1e5
+    x[rng.integers(0, n, 5)] = np.nan
+    x[rng.integers(0, n, 5)] = -np.inf
+    key = host_col(k, rng.random(n) >= 0.02)
+    assert_parity([key], [(host_col(x, rng.random(n) >= 0.05), [(AGG["VARIANCE"], 1), (AGG["STD"], 0), (AGG["COUNT_VALID"], 1)]),
+                          (host_col(rng.integers(0, 50, n).astype(np.uint16)), [(AGG["VARIANCE"], 1), (AGG["MEAN"], 1)])], 1)
