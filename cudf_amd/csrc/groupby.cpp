@@ -1897,8 +1897,9 @@ int64_t groupby_call::aggregate_global()
   // overflows costs the rows processed before the rebuild
   uint64_t cap = std::max<uint64_t>(64, next_pow2(uint64_t(est_ * (est_low_ ? 10.4 : 2.6)) + 1));
   cap = std::min(cap, max_cap);
-  int32_t* d_flags = S->get<int32_t>(4);  // [0] overflow, [1..2] special occupancy
+  int32_t* d_flags = S->get<int32_t>(4);  // [0] overflow, [1..2] special occupancy, [3] groups (small tables)
   uint32_t* block_counts = nullptr;
+  uint32_t* map          = nullptr;
   int retries = 0;
   int64_t G   = -1;
   size_t const table_mark = S->mark();
@@ -1920,14 +1921,24 @@ int64_t groupby_call::aggregate_global()
     T->mark(3);
     MIG_HIP_TRY(hipGetLastError());
 
-    int64_t nb   = (int64_t(cap) + 2 + SCAN_TILE - 1) / SCAN_TILE;
-    block_counts = S->get<uint32_t>(nb + 1);
-    launch_count_occupied(dP, p, block_counts, stream_);
-    launch_scan_blocks(block_counts, nb, block_counts + nb, stream_);
     auto* h_flags = reinterpret_cast<uint32_t*>(pin + 2 * sizeof(gb_params));
-    MIG_HIP_TRY(hipMemcpyAsync(h_flags, d_flags, 4, hipMemcpyDeviceToHost, stream_));
-    MIG_HIP_TRY(hipMemcpyAsync(h_flags + 1, block_counts + nb, 4, hipMemcpyDeviceToHost, stream_));
-    MIG_HIP_TRY(hipStreamSynchronize(stream_));
+    if (cap <= COMPACT_SMALL) {
+      map = S->get<uint32_t>(cap + 2);
+      launch_compact_small(dP, map, reinterpret_cast<uint32_t*>(d_flags + 3), stream_);
+      MIG_HIP_TRY(hipMemcpyAsync(h_flags + 1, d_flags, 16, hipMemcpyDeviceToHost, stream_));
+      MIG_HIP_TRY(hipStreamSynchronize(stream_));
+      h_flags[0] = h_flags[1];
+      h_flags[1] = h_flags[4];
+    } else {
+      map          = nullptr;
+      int64_t nb   = (int64_t(cap) + 2 + SCAN_TILE - 1) / SCAN_TILE;
+      block_counts = S->get<uint32_t>(nb + 1);
+      launch_count_occupied(dP, p, block_counts, stream_);
+      launch_scan_blocks(block_counts, nb, block_counts + nb, stream_);
+      MIG_HIP_TRY(hipMemcpyAsync(h_flags, d_flags, 4, hipMemcpyDeviceToHost, stream_));
+      MIG_HIP_TRY(hipMemcpyAsync(h_flags + 1, block_counts + nb, 4, hipMemcpyDeviceToHost, stream_));
+      MIG_HIP_TRY(hipStreamSynchronize(stream_));
+    }
     if (h_flags[0] == 0) {
       G = h_flags[1];
       break;
@@ -1946,8 +1957,10 @@ int64_t groupby_call::aggregate_global()
     else launch_second_pass(dP, p, num_cus, stream_);
   }
   T->mark(5);
-  uint32_t* map = S->get<uint32_t>(std::max<int64_t>(G, 1));
-  launch_compact(dP, p, block_counts, map, stream_);
+  if (map == nullptr) {
+    map = S->get<uint32_t>(std::max<int64_t>(G, 1));
+    launch_compact(dP, p, block_counts, map, stream_);
+  }
   T->mark(6);
 
   alloc_outputs(G, G, false);

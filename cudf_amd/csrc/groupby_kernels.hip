@@ -1627,6 +1627,39 @@ void launch_compact(gb_params const* dP, gb_params const& hP, uint32_t const* bl
   hipLaunchKernelGGL(k_compact, dim3(nb), dim3(BLOCK), 0, s, dP, block_offsets, map);
 }
 
+// Both steps and the scan between them for a small table, by one workgroup:
+// map[g] = slot of dense group g, *total = groups.
+__global__ void __launch_bounds__(1024) k_compact_small(gb_params const* __restrict__ Pp, uint32_t* map, uint32_t* total)
+{
+  __shared__ uint32_t wave_tot[1024 / 64];
+  gb_params const& P   = *Pp;
+  uint32_t const slots = uint32_t(P.cap) + 2u;
+  uint32_t const per   = (slots + 1023u) / 1024u;  // at most COMPACT_SMALL / 1024 + 1
+  uint32_t const b     = threadIdx.x * per;
+  int const wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  uint32_t occ = 0;  // bit j: slot b + j
+  for (uint32_t j = 0; j < per; j++)
+    if (b + j < slots && slot_occupied(P, b + j)) occ |= 1u << j;
+  uint32_t const mine = uint32_t(__popc(occ));
+  uint32_t incl       = mine;
+  for (int o = 1; o < 64; o <<= 1) {
+    uint32_t const y = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += y;
+  }
+  if (lane == 63) wave_tot[wave] = incl;
+  __syncthreads();
+  uint32_t at = incl - mine;
+  for (int w = 0; w < wave; w++) at += wave_tot[w];
+  for (uint32_t j = 0; j < per; j++)
+    if ((occ >> j) & 1u) map[at++] = b + j;
+  if (threadIdx.x == 1023) *total = at;
+}
+
+void launch_compact_small(gb_params const* dP, uint32_t* map, uint32_t* total, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_compact_small, dim3(1), dim3(1024), 0, s, dP, map, total);
+}
+
 // ---------------------------------------------------------------------------
 // dense outputs: keys and aggregation results for group g = blockIdx*BLOCK+tid
 __device__ __forceinline__ uint64_t field_bits(field_desc const& F, int64_t slot)

@@ -365,6 +365,10 @@ void launch_scan_blocks(uint32_t* block_counts, int64_t nblocks, uint32_t* total
 // Writes map[g] = slot of dense group g, in slot order.
 void launch_compact(gb_params const* dP, gb_params const& hP, uint32_t const* block_offsets,
                     uint32_t* map, hipStream_t s);
+// All of that in one launch for a table of at most COMPACT_SMALL slots (three
+// launches and two copies of a call with few groups: about 20 us).
+constexpr uint64_t COMPACT_SMALL = 16384;
+void launch_compact_small(gb_params const* dP, uint32_t* map, uint32_t* total, hipStream_t s);
 // Writes keys (inline table) or representative rows (general table) and all
 // aggregation results of the G dense groups.
 void launch_outputs(gb_params const* dP, gb_params const& hP, uint32_t const* map, int64_t G,
