@@ -1547,12 +1547,16 @@ int64_t groupby_call::aggregate_partitioned()
     // partition buffers
     size_t part_bytes = 0;
     R.keysB  = S->get<uint64_t>(rowsB);
-    R.flagsB = S->get<uint8_t>(rowsB);
-    part_bytes += 9 * size_t(rowsB);
+    // a flags byte per record only where one can be set: value columns with
+    // nulls, or null keys kept as a group
+    bool const flagged = flag_bit > 0 || (p.key_mode == KM_INLINE && p.keys[0].mask != nullptr && !p.skip_null_keys);
+    R.flagsA = R.flagsB = nullptr;
+    if (flagged) R.flagsB = S->get<uint8_t>(rowsB);
+    part_bytes += (flagged ? 9 : 8) * size_t(rowsB);
     if (R.two_level) {
-      R.keysA  = S->get<uint64_t>(rowsA);
-      R.flagsA = S->get<uint8_t>(rowsA);
-      part_bytes += 9 * size_t(rowsA);
+      R.keysA = S->get<uint64_t>(rowsA);
+      if (flagged) R.flagsA = S->get<uint8_t>(rowsA);
+      part_bytes += (flagged ? 9 : 8) * size_t(rowsA);
     }
     R.general_hashed = hashed ? 1 : 0;
     R.rowsA = R.rowsB = nullptr;

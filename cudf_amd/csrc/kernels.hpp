@@ -261,7 +261,7 @@ struct rpa_params {
   int32_t* cap_overflow;
   uint64_t* keysA;
   uint64_t* keysB;
-  uint8_t* flagsA;
+  uint8_t* flagsA;  // null when no record has a flag (no nulls the path keeps)
   uint8_t* flagsB;
   uint8_t* valsA[MAX_VALS];
   uint8_t* valsB[MAX_VALS];

@@ -97,6 +97,8 @@ struct acc_plan {
   int32_t ncols;
   int32_t nfields;
   bool wide_f32;
+  bool flagged;  // else `flags` names a byte of the keys, masked to 0
+  uint32_t flag_mask;
   int32_t key_storage;
   int32_t count_all_off;
   uint32_t cd_lane;     // lane i < ncols: storage | (flag bit + 1) << 8 | first field << 16 | end << 24
@@ -117,7 +119,9 @@ __device__ __forceinline__ acc_plan load_plan(gb_params const& P, rpa_params con
   A.key_storage   = P.key_storage;
   A.count_all_off = R.count_all_off;
   A.keys          = gp(static_cast<uint64_t const*>(R.keysB));
-  A.flags         = gp(static_cast<uint8_t const*>(R.flagsB));
+  A.flagged       = R.flagsB != nullptr;
+  A.flag_mask     = A.flagged ? 0xffu : 0u;
+  A.flags         = gp(A.flagged ? static_cast<uint8_t const*>(R.flagsB) : reinterpret_cast<uint8_t const*>(R.keysB));
   A.rows          = gp(static_cast<uint32_t const*>(R.rowsB));
   int const lane  = int(threadIdx.x & 63);
   int const i     = lane < A.ncols ? lane : 0;
@@ -199,7 +203,7 @@ __device__ __forceinline__ void chunk_load(acc_plan const& A, int64_t r0, int64_
   for (int k = 0; k < RPA_CACHED; k++) {  // rows past the bin read its last row (e > r0 - tid)
     int64_t const r  = r0 + int64_t(k) * RPA_AGG_BLOCK;
     int64_t const rc = r < e ? r : e - 1;
-    fl[k]            = A.flags[rc];
+    fl[k]            = uint8_t(A.flags[A.flagged ? rc : 0] & A.flag_mask);
     in.key[k]        = A.keys[rc];
     if (KM == KF_HASHED) in.row[k] = A.rows[rc];
   }

@@ -330,6 +330,11 @@ __global__ void __launch_bounds__(RPA_SCATTER_BLOCK) __attribute__((amdgpu_waves
   auto* sbins     = reinterpret_cast<uint16_t*>(stage + R.stage_bin_off);
   auto* srows     = reinterpret_cast<uint32_t*>(stage + R.stage_row_off);  // hashed general keys only
   bool const hashed     = R.general_hashed != 0;
+  // without flags every row reads one byte of its keys and masks it (a branch
+  // around the load would separate the rows' loads)
+  bool const flagged      = R.flagsB != nullptr;
+  uint8_t const flag_mask = flagged ? 0xff : 0;
+  uint8_t const* in_flags = flagged ? R.flagsA : reinterpret_cast<uint8_t const*>(R.keysA);
   uint64_t* const okeys = (SECOND || !R.two_level) ? R.keysB : R.keysA;
   uint8_t* const oflags = (SECOND || !R.two_level) ? R.flagsB : R.flagsA;
   uint32_t* const orows = (SECOND || !R.two_level) ? R.rowsB : R.rowsA;
@@ -379,7 +384,7 @@ __global__ void __launch_bounds__(RPA_SCATTER_BLOCK) __attribute__((amdgpu_waves
       if (row >= r1) continue;
       uint32_t h;
       if constexpr (SECOND) {
-        kf[k] = gp(static_cast<uint8_t const*>(R.flagsA))[row];
+        kf[k] = gp(in_flags)[flagged ? row : 0] & flag_mask;
         kb[k] = gp(static_cast<uint64_t const*>(R.keysA))[row];
         if (hashed) rw[k] = gp(static_cast<uint32_t const*>(R.rowsA))[row];
         h     = record_hash(P, kb[k], kf[k]);
@@ -465,7 +470,7 @@ __global__ void __launch_bounds__(RPA_SCATTER_BLOCK) __attribute__((amdgpu_waves
     }
 #pragma unroll
     for (int k = 0; k < RPA_MAX_RPT; k++)
-      if (lp[k] >= 0) sflags[lp[k]] = kf[k];
+      if (flagged && lp[k] >= 0) sflags[lp[k]] = kf[k];
     lds_barrier();
     // ---- write bin runs
     int const total = int(toff[fan]);
@@ -474,7 +479,7 @@ __global__ void __launch_bounds__(RPA_SCATTER_BLOCK) __attribute__((amdgpu_waves
       if (base[b] == NO_BASE) continue;
       int64_t const dst = int64_t(base[b]) + (lp - int(toff[b]));
       gp(okeys)[dst]    = skeys[lp];
-      gp(oflags)[dst]   = sflags[lp];
+      if (flagged) gp(oflags)[dst] = sflags[lp];
       if (hashed) gp(orows)[dst] = srows[lp];
       for (int i = 0; i < ncols; i++) {
         int const v       = R.plan_col[i];
