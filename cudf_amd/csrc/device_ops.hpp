@@ -235,18 +235,21 @@ __device__ __forceinline__ void row_hash2(dcol const* cols, int ncols, int64_t r
   }
 }
 
-__device__ __forceinline__ bool elem_equal(dcol const& c, int64_t a, int64_t b)
+// Whether row a of `c` equals row b of `o`, a column of the same storage.
+__device__ __forceinline__ bool elem_equal(dcol const& c, int64_t a, dcol const& o, int64_t b)
 {
-  bool const va = dcol_valid(c, a), vb = dcol_valid(c, b);
+  bool const va = dcol_valid(c, a), vb = dcol_valid(o, b);
   if (!va || !vb) return va == vb;
   if (c.storage == ST_STRING) {
     int64_t ab, ae, bb, be;
     str_span(c, a, ab, ae);
-    str_span(c, b, bb, be);
-    return ae - ab == be - bb && bytes_equal(gp(c.data) + ab, gp(c.data) + bb, ae - ab);
+    str_span(o, b, bb, be);
+    return ae - ab == be - bb && bytes_equal(gp(c.data) + ab, gp(o.data) + bb, ae - ab);
   }
-  return load_fixed_bits(c, a) == load_fixed_bits(c, b);
+  return load_fixed_bits(c, a) == load_fixed_bits(o, b);
 }
+
+__device__ __forceinline__ bool elem_equal(dcol const& c, int64_t a, int64_t b) { return elem_equal(c, a, c, b); }
 
 __device__ __forceinline__ bool rows_equal(gb_params const& P, int64_t a, int64_t b)
 {

@@ -702,6 +702,7 @@ class groupby_call {
   int64_t aggregate_partitioned();
   int64_t aggregate_hot_split();
   bool partitionable();
+  bool verify_hashed(rpa_params const* dR, rpa_params const& R);
   bool partitioning_pays();
   bool few_groups();
   int64_t aggregate_global();
@@ -1343,6 +1344,28 @@ bool groupby_call::partitioning_pays()
   return N >= 300'000 && (atomics >= 3 || est_ <= 1024.0) && !straggler;
 }
 
+// The exact check of the hashed form against the gathered key columns.
+bool groupby_call::verify_hashed(rpa_params const* dR, rpa_params const& R)
+{
+  key_columns out{};
+  for (int i = 0; i < num_keys_; i++) {
+    mig_column const& c = res_->keys[size_t(i)].col;
+    out.col[i].storage  = storage_of(keys_[i].type_id);
+    out.col[i].data     = static_cast<uint8_t const*>(c.data);
+    out.col[i].mask     = c.null_mask;
+    out.col[i].offsets  = c.offsets;  // int32
+  }
+  launch_rpa_verify(dP, dR, out, R.rec_count, stream_);
+  MIG_HIP_TRY(hipGetLastError());
+  auto* h = reinterpret_cast<uint64_t*>(pin + 2 * sizeof(gb_params));
+  h[1]    = 0;
+  MIG_HIP_TRY(hipMemcpyAsync(h, R.verified, 8, hipMemcpyDeviceToHost, stream_));
+  MIG_HIP_TRY(hipMemcpyAsync(h + 1, R.verify_failed, 4, hipMemcpyDeviceToHost, stream_));
+  MIG_HIP_TRY(hipStreamSynchronize(stream_));
+  stats_[STAT_VERIFIED_PAIRS] = double(h[0]);
+  return uint32_t(h[1]) == 0;
+}
+
 // Radix-partitioned LDS aggregation for high cardinality: returns the number
 // of groups, or -1 when the path does not apply (or its bins overflowed three
 // times) and the device-wide table takes the call.
@@ -1607,28 +1630,12 @@ int64_t groupby_call::aggregate_partitioned()
     launch_rpa_aggregate(dP, dR, R, p.key_mode == KM_GENERAL ? (hashed ? 2 : 1) : 0, 0, B, stream_);
     T->mark(13);
     MIG_HIP_TRY(hipGetLastError());
-    // the hashed form compares every record with its representative before
-    // the results are read back (a no-op launch for the other forms)
-    if (hashed) launch_rpa_verify(dP, dR, R.rec_count, stream_);
-    MIG_HIP_TRY(hipGetLastError());
     auto* h = reinterpret_cast<uint64_t*>(pin + 2 * sizeof(gb_params));
-    h[2] = 0;
-    h[3] = 0;
     MIG_HIP_TRY(hipMemcpyAsync(h, R.group_counter, 8, hipMemcpyDeviceToHost, stream_));
     MIG_HIP_TRY(hipMemcpyAsync(h + 1, d_small, 8, hipMemcpyDeviceToHost, stream_));
-    if (hashed) {
-      MIG_HIP_TRY(hipMemcpyAsync(h + 2, R.verified, 8, hipMemcpyDeviceToHost, stream_));
-      MIG_HIP_TRY(hipMemcpyAsync(h + 3, R.verify_failed, 4, hipMemcpyDeviceToHost, stream_));
-    }
     MIG_HIP_TRY(hipStreamSynchronize(stream_));
     uint32_t const groups_overflow = uint32_t(h[1]), bins_overflow = uint32_t(h[1] >> 32);
-    bool const verify_failed = hashed && !bins_overflow && groups_overflow == 0 && uint32_t(h[3]) != 0;
-    stats_[STAT_VERIFIED_PAIRS] = double(h[2]);
-    if (verify_failed) {  // two different keys met with equal words: compare key rows instead
-      release_outputs();
-      hashed = false;
-      stats_[STAT_RETRIES] += 1;
-    } else if (bins_overflow) {  // a speculative bin filled up: the same bins, laid out exactly
+    if (bins_overflow) {  // a speculative bin filled up: the same bins, laid out exactly
       release_outputs();
       speculative = false;
       stats_[STAT_RETRIES] += 1;
@@ -1638,6 +1645,14 @@ int64_t groupby_call::aggregate_partitioned()
       for (auto& rc : res_->results)
         for (auto& c : rc) c.col.size = int32_t(G);
       if (p.key_mode == KM_GENERAL) gather_general_keys(R.out_rep, G);
+      // the hashed form compares every record with its group's key
+      if (hashed && !verify_hashed(dR, R)) {  // two different keys met with equal words: compare key rows instead
+        release_outputs();
+        hashed = false;
+        G      = -1;
+        stats_[STAT_RETRIES] += 1;
+        continue;
+      }
       stats_[STAT_STRATEGY] = MIG_STRATEGY_PARTITIONED;
       stats_[STAT_CAPACITY] = double(B);
       stats_[STAT_RETRIES] += bin_attempts;

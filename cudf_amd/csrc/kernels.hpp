@@ -276,10 +276,11 @@ struct rpa_params {
   // in rowsA / rowsB, and bins compare words instead of key rows.  A bin slot's
   // representative row is rep_rows[bin * rep_stride + slot]; rec_slot[row]
   // (input row; 0xFFFFFFFF for dropped rows and representatives) receives the
-  // slot of the row's group, and k_rpa_verify compares every such row's key
-  // row with its representative's exactly afterwards, in row order (any
-  // difference reruns the call with general_hashed = 0, which compares key
-  // rows while probing).
+  // slot of the row's group; once the group's result row is known it takes the
+  // representative's place in rep_rows, and k_rpa_verify compares every such
+  // row's key row with that row of the gathered key columns exactly, in row
+  // order (any difference reruns the call with general_hashed = 0, which
+  // compares key rows while probing).
   int32_t general_hashed;
   int32_t stage_row_off;
   int64_t rep_stride;
@@ -497,6 +498,10 @@ void launch_rpa_scatter2(gb_params const* dP, rpa_params const* dR, rpa_params c
 void launch_rpa_aggregate(gb_params const* dP, rpa_params const* dR, rpa_params const& hR, int key_form,
                           int64_t bin_begin, int64_t bin_end, hipStream_t s);
 // exact key comparison of the (row, representative) pairs of the hashed form
-void launch_rpa_verify(gb_params const* dP, rpa_params const* dR, int64_t records, hipStream_t s);
+struct key_columns {  // the result's key columns
+  dcol col[MAX_KEYS];
+};
+void launch_rpa_verify(gb_params const* dP, rpa_params const* dR, key_columns const& out, int64_t records,
+                       hipStream_t s);
 
 }  // namespace mig

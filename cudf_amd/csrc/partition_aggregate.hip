@@ -612,9 +612,11 @@ __global__ void __launch_bounds__(RPA_AGG_BLOCK) __attribute__((amdgpu_waves_per
     bool const kvalid   = slot != S;
     if (live && !in_range) astore(R.overflow, 1);
     if (KM == KF_HASHED) {  // keys are gathered from the representative rows afterwards
-      if (in_range)
-        gp(R.out_rep)[pos] = __hip_atomic_load(gp(R.rep_rows) + rbase + slot, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
+      if (in_range) {
+        auto const rep     = gp(R.rep_rows) + rbase + slot;
+        gp(R.out_rep)[pos] = __hip_atomic_load(rep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *rep               = uint32_t(pos);  // for the verification
+      }
     } else if (KM == KF_GENERAL) {
       if (in_range) gp(R.out_rep)[pos] = uint32_t(tkeys[slot]);
     } else {
@@ -726,14 +728,16 @@ void launch_rpa_aggregate(gb_params const* dP, rpa_params const* dR, rpa_params 
   else launch_aggregate_form<KF_INLINE>(dP, dR, hR, bin_begin, bin_end, s);
 }
 
-// Exact comparison of every record of the hashed form with its group's
-// representative: rows whose group was found by equal 64-bit words must also
-// have equal keys (nulls equal, NaN equal NaN, -0.0 equal 0.0, strings
-// byte-wise), otherwise verify_failed is set and the call is redone comparing
-// key rows.  Rows are visited in input order, so a row's own keys are read
-// sequentially and only the representatives' are random reads.
+// Exact comparison of every record of the hashed form with its group's key:
+// rows whose group was found by equal 64-bit words must also have equal keys
+// (nulls equal, NaN equal NaN, -0.0 equal 0.0, strings byte-wise), otherwise
+// verify_failed is set and the call is redone comparing key rows.  Rows are
+// visited in input order, so a row's own keys are read sequentially; the
+// group's are read at its row of the finished key columns, which are random
+// reads into a tenth of the memory that its first input row's would touch
+// (10M int + string rows, 900K groups: 786 us with those, 671 us now).
 __global__ void __launch_bounds__(256) k_rpa_verify(gb_params const* __restrict__ Pp, rpa_params const* __restrict__ Rp,
-                                                    int64_t records)
+                                                    key_columns out, int64_t records)
 {
   __shared__ uint32_t block_count;
   gb_params const& P  = *Pp;
@@ -745,11 +749,9 @@ __global__ void __launch_bounds__(256) k_rpa_verify(gb_params const* __restrict_
   for (int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x; r < records; r += int64_t(gridDim.x) * 256) {
     uint32_t const gs = gp(R.rec_slot)[r];
     if (gs == 0xffffffffu) continue;  // a dropped row, or a representative
-    uint32_t const row = uint32_t(r);
-    uint32_t const rep = __hip_atomic_load(gp(R.rep_rows) + gs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (rep == row) continue;
+    int64_t const g = int64_t(gp(R.rep_rows)[gs]);
     count++;
-    bad |= !rows_equal(P, int64_t(row), int64_t(rep));
+    for (int c = 0; c < P.num_keys; c++) bad |= !elem_equal(P.keys[c], r, out.col[c], g);
   }
   if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) astore(R.verify_failed, 1);
   if (count) __hip_atomic_fetch_add(&block_count, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -758,12 +760,13 @@ __global__ void __launch_bounds__(256) k_rpa_verify(gb_params const* __restrict_
     __hip_atomic_fetch_add(gp(R.verified), (unsigned long long)block_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-void launch_rpa_verify(gb_params const* dP, rpa_params const* dR, int64_t records, hipStream_t s)
+void launch_rpa_verify(gb_params const* dP, rpa_params const* dR, key_columns const& out, int64_t records,
+                       hipStream_t s)
 {
   if (records <= 0) return;
   int64_t blocks = (records + 255) / 256;
   if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(k_rpa_verify, dim3(blocks), dim3(256), 0, s, dP, dR, records);
+  hipLaunchKernelGGL(k_rpa_verify, dim3(blocks), dim3(256), 0, s, dP, dR, out, records);
 }
 
 }  // namespace mig
