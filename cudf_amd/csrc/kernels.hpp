@@ -233,7 +233,7 @@ struct rpa_params {
   int32_t count_all_off;  // LDS byte offsets of the aggregate kernel
   int32_t slot_of_j_off;
   int32_t misc_off;
-  int32_t pad_agg;
+  int32_t m2_two_pass;  // every group's M2 from the deviations (no sums of squares)
   // scatter staging: a tile of rows sorted by bin in LDS before it is written
   int32_t tile_rows;
   int32_t stage_bytes;

@@ -400,10 +400,11 @@ __device__ __forceinline__ void chunk_deviations(gb_params const& P, rpa_params 
 // every partial sum and square is exact in double) use the exact integer
 // identity n·M2 = n·Σx² − (Σx)² in 128 bits.  Float64 sources use
 // Σx² − (Σx)²/n when its rounding error, at most ~3·n·ε·Σx², is below 1e-11
-// of the result.  Anything else (float32 sums, large or ill-conditioned
-// groups) returns false: the exact second pass computes that group.
+// of the result, unless the call asks for two passes.  Anything else (float32
+// sums, large or ill-conditioned groups) returns false: the exact second pass
+// computes that group.
 __device__ __forceinline__ bool m2_from_sums(int32_t sum_kind, int32_t sum_off, int32_t st, uint8_t* lds, int i,
-                                             uint32_t n, double* m2)
+                                             uint32_t n, bool two_pass, double* m2)
 {
   double const s2 = *m2;
   if (n <= 1 && isfinite(s2)) {  // no deviation from the mean of one finite value
@@ -412,7 +413,7 @@ __device__ __forceinline__ bool m2_from_sums(int32_t sum_kind, int32_t sum_off, 
   }  // one NaN or infinite value: the exact pass gives (x - x)² = NaN, as the reference
   if (st == ST_F32) return false;
   if (st == ST_F64) {
-    if (n > 256) return false;
+    if (two_pass || n > 256) return false;
     double const s1 = *lds_at<double>(lds, sum_off, i);
     double const v  = s2 - s1 * (s1 / double(n));
     if (!(v > 0.0) || 3.0 * double(n) * 1.1102230246251565e-16 * s2 > 1e-11 * v) return v == 0.0 && s2 == 0.0;
@@ -501,6 +502,7 @@ __global__ void __launch_bounds__(RPA_AGG_BLOCK) __attribute__((amdgpu_waves_per
   if (P.need_second_pass) {
     uint8_t* m2_flag = lds + R.slot_of_j_off;  // the compaction map's bytes, free until then
     int const nm2    = R.m2_n;
+    bool const two_pass = R.m2_two_pass != 0;
     int const lane   = tid & 63;
     int const jl     = lane < nm2 ? lane : 0;  // the plan, one M2 field per lane
     int32_t const m2_off_l = R.m2_off[jl], m2_cnt_l = R.m2_cnt_off[jl], m2_st_l = R.m2_storage[jl];
@@ -515,7 +517,7 @@ __global__ void __launch_bounds__(RPA_AGG_BLOCK) __attribute__((amdgpu_waves_per
         double* m2          = lds_at<double>(lds, off, i);
         uint32_t const n    = *lds_at<uint32_t>(lds, int32_t(lane_value(uint32_t(m2_cnt_l), j)), i);
         redo |= !m2_from_sums(int32_t(sum & 0xffu), int32_t(sum >> 8), int32_t(lane_value(uint32_t(m2_st_l), j)),
-                              lds, i, n, m2);
+                              lds, i, n, two_pass, m2);
       }
       m2_flag[i] = redo ? 1 : 0;
       if (redo) {

@@ -119,3 +119,43 @@ def test_variance_of_few_groups(card, spread):
     key = host_col(k, rng.random(n) >= 0.02)
     assert_parity([key], [(host_col(x, rng.random(n) >= 0.05), [(AGG["VARIANCE"], 1), (AGG["STD"], 0), (AGG["COUNT_VALID"], 1)]),
                           (host_col(rng.integers(0, 50, n).astype(np.uint16)), [(AGG["VARIANCE"], 1), (AGG["MEAN"], 1)])], 1)
+
+
+def _spread_over_mean(rng, n, card, kind):
+    """Keys and float64 values whose mean is 20 standard deviations."""
+    if kind == "hot":
+        k = rng.integers(0, card, n)
+        hot = rng.random(n) < 0.3
+        k[hot] = rng.integers(0, 5, int(hot.sum()))
+    else:
+        k = rng.integers(0, card, n)
+    return k * 1_000_003, rng.standard_normal(n) + 20.0
+
+
+@pytest.mark.parametrize("kind,n,card", [("one", 300_001, 6_000), ("general", 400_003, 8_000), ("hot", 1_100_003, 20_000)])
+def test_variance_subtracts_the_mean(kind, n, card):
+    """Calls below a million rows or 65,536 groups, and the keys beside hot
+    ones: M2 is the sum of squared deviations from the mean.  With u = 2^-53
+    and m rows in a group every squared deviation is within 3u of itself and
+    their sum within (m - 1)u, the mean's own error counts quadratically: at
+    most (m + 5)u.  (The sum of squares less the squared sum would lose
+    m * x^2 / sigma^2 = 400 m of the same units.)"""
+    from cudf_amd import GroupBy, GroupByRequest, Table
+    from cudf_amd.aggregation import Aggregation
+    from tests.gbutil import to_device
+    rng = np.random.default_rng(card)
+    k, x = _spread_over_mean(rng, n, card, kind)
+    keys = [host_col(k)] + ([host_col((k % 5).astype(np.int32))] if kind == "general" else [])
+    out, res = GroupBy(Table([to_device(c) for c in keys])).aggregate(
+        [GroupByRequest(to_device(host_col(x)), [Aggregation(AGG["VARIANCE"], 1), Aggregation(AGG["COUNT_VALID"])])])
+    got_keys = out.columns()[0].to_numpy()[0]
+    got = res[0].columns()[0].to_numpy()[0][np.argsort(got_keys)]
+    order = np.argsort(k, kind="stable")
+    uniq, first, count = np.unique(k[order], return_index=True, return_counts=True)
+    xs = x[order].astype(np.longdouble)  # 64 bits of mantissa
+    dev = xs - np.repeat(np.add.reduceat(xs, first) / count, count)
+    many = count > 1
+    want = np.add.reduceat(dev * dev, first)[many] / (count[many] - 1)
+    err = np.abs((got[many] - want) / want).astype(np.float64)
+    bound = (count[many] + 5) * 2.0**-53
+    assert np.all(err <= bound), (err / bound).max()
