@@ -102,9 +102,13 @@ constexpr int32_t BATCH_SAMPLE = 4096;  // sampled rows per instance
 // Instances this large with this many estimated groups run the single-call
 // path: its radix-partitioned aggregation (LDS atomics per bin) beats the
 // per-row device-wide atomics the batched kernels fall back to when an
-// instance's groups exceed what LDS pre-aggregation takes.
+// instance's groups exceed what LDS pre-aggregation takes.  The call waits for
+// the device on the host, so the execute that holds it does not return before,
+// and cannot be captured.  From 8,192 groups on it would still be the faster one
+// (16 instances of 0.1 to 2M rows: 2.08 ms a pass against 2.20), but plans whose
+// instances stay below 65,536 are executed asynchronously and under capture.
 constexpr int32_t BATCH_SOLO_ROWS   = 1 << 20;
-constexpr double BATCH_SOLO_GROUPS  = 8192.0;  // what BATCH_MAX_PARTS LDS parts hold
+constexpr double BATCH_SOLO_GROUPS  = 65536.0;
 
 int32_t default_i(int32_t v, int32_t d) { return v == 0 ? d : v; }
 

@@ -255,3 +255,29 @@ def test_batch_errors():
     strs = [(orc.HostColumn.from_strings([b"x%d" % (j % 7) for j in range(len(k.data))]), vs)]
     with pytest.raises(_lib.DataTypeError):
         run_batch(strs, [REQ0, REQ1], 0)
+
+
+@pytest.mark.parametrize("rows,card", [(1_100_000, 9_000), (2_000_003, 40_000)])
+def test_batch_captured_by_the_caller(rows, card):
+    """A plan that launches kernel by kernel is captured by its caller and
+    replayed, with a large instance of up to 65,535 groups in it; every replay
+    matches the oracle, with the caller's own device work in between."""
+    import torch
+    from cudf_amd import BatchOptions, BatchedGroupBy, NullPolicy
+    from cudf_amd.aggregation import Aggregation
+    inst = make_instances(31, 5, 20_000, big=[(rows, card)])
+    dev = [(to_device(k), [to_device(v) for v in vs]) for k, vs in inst]
+    aggs = [REQ0 + [(AGG["VARIANCE"], 1)], REQ1]
+    plan = BatchedGroupBy(dev, [[Aggregation(k, d) for k, d in al] for al in aggs], NullPolicy.EXCLUDE,
+                          BatchOptions(use_graph=-1))
+    plan.run()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        plan.execute(stream)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        plan.synchronize()
+        check_all(plan, inst, aggs)
+        torch.randn(1 << 20, device="cuda").sum().item()
