@@ -1830,7 +1830,7 @@ int64_t groupby_call::aggregate_hot_split()
   uint32_t* block_counts = S->get<uint32_t>(nb + 1);
   launch_count_occupied(dP, p, block_counts, stream_);
   launch_scan_blocks(block_counts, nb, block_counts + nb, stream_);
-  if (p.need_second_pass) launch_second_pass_lds(dP, p, blocks, stream_);
+  if (p.need_second_pass) launch_second_pass_lds(dP, p, blocks, true, stream_);  // at most half the slots
   auto* h = reinterpret_cast<uint32_t*>(pin + 2 * sizeof(gb_params));
   MIG_HIP_TRY(hipMemcpyAsync(h, d_flags, 16, hipMemcpyDeviceToHost, stream_));
   MIG_HIP_TRY(hipMemcpyAsync(h + 4, block_counts + nb, 4, hipMemcpyDeviceToHost, stream_));
@@ -1980,7 +1980,8 @@ int64_t groupby_call::aggregate_global()
 
   T->mark(4);
   if (p.need_second_pass) {
-    if (lds_blocks > 0) launch_second_pass_lds(dP, p, lds_blocks, stream_);
+    // by value, what is outside the sampled range is rare
+    if (lds_blocks > 0) launch_second_pass_lds(dP, p, lds_blocks, p.lds_direct || G <= p.lds_fill, stream_);
     else launch_second_pass(dP, p, num_cus, stream_);
   }
   T->mark(5);

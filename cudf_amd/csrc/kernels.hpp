@@ -356,7 +356,8 @@ void launch_aggregate(gb_params const* dP, gb_params const& hP, int num_cus, hip
 // Low-cardinality form of launch_aggregate / launch_second_pass (inline keys,
 // hP.lds_bytes > 0): `blocks` workgroups pre-aggregate their rows in LDS.
 void launch_aggregate_lds(gb_params const* dP, gb_params const& hP, int64_t blocks, hipStream_t s);
-void launch_second_pass_lds(gb_params const* dP, gb_params const& hP, int64_t blocks, hipStream_t s);
+// `all_fit`: the LDS tables hold every group.
+void launch_second_pass_lds(gb_params const* dP, gb_params const& hP, int64_t blocks, bool all_fit, hipStream_t s);
 void launch_second_pass(gb_params const* dP, gb_params const& hP, int num_cus, hipStream_t s);
 // Occupancy scan: block_counts has ceil((cap+2)/SCAN_TILE) entries.
 constexpr int SCAN_TILE = 4096;

@@ -159,3 +159,28 @@ def test_variance_subtracts_the_mean(kind, n, card):
     err = np.abs((got[many] - want) / want).astype(np.float64)
     bound = (count[many] + 5) * 2.0**-53
     assert np.all(err <= bound), (err / bound).max()
+
+
+def test_variance_when_the_hot_key_comes_last():
+    """Zipf(2) keys: more groups than the estimate sized the LDS tables for,
+    and the key of most rows in the last slots of the device-wide table.  Its
+    rows must not queue up on one address (37 ms when they do, 0.1 ms else)."""
+    from cudf_amd import _lib
+    from oracle import oracle as orc
+    rng = np.random.default_rng(3)
+    n, card = 5_000_003, 2_500_000
+    w = np.arange(1, card + 1, dtype=np.float64) ** -2.0
+    rank = np.minimum(np.searchsorted(np.cumsum(w) / w.sum(), rng.random(n)), card - 1)
+    candidates = np.arange(1, 200_000, dtype=np.int64) << 40
+    slot = orc.hash_rows([host_col(candidates)]).astype(np.int64) & (2**14 - 1)
+    ids = rng.permutation(card).astype(np.int64) * 1_000_003
+    ids[0] = candidates[slot >= 2**14 - 4][0]
+    v = host_col(rng.standard_normal(n))
+    _lib.set_phase_timing(True)
+    try:
+        assert_parity([host_col(ids[rank])], [(v, [(AGG["VARIANCE"], 1), (AGG["MEAN"], 1)])])
+        st = _stats()
+    finally:
+        _lib.set_phase_timing(False)
+    assert st["lds_preagg"] == 1.0 and st["groups"] > 2.6 * st["est_groups"], st
+    assert st["t_second_pass_ms"] < 4.0, st
