@@ -705,6 +705,7 @@ class groupby_call {
   bool verify_hashed(rpa_params const* dR, rpa_params const& R);
   bool partitioning_pays();
   bool high_cardinality() const;
+  int32_t lds_slots(bool& direct);
   bool few_groups();
   int64_t aggregate_global();
   int32_t lds_most_slots();
@@ -1686,15 +1687,45 @@ int32_t groupby_call::lds_most_slots()
   return (LDS_PREAGG_BUDGET / std::max(row_bytes, m2_bytes) - LDS_EXTRA_SLOTS - 16) & ~63;
 }
 
-// Whether the LDS partial tables hold the (estimated) groups of a fixed-width
-// key: at least 1.45x the estimate's slots, or a slot for every key of the
-// sampled range.
+// Slots of the LDS partial tables for the (estimated) groups of a fixed-width
+// key, 0 when they don't hold them or don't pay.  A slot for every key of the
+// sampled range (`direct`), else a third of the slots filled (the longest probe
+// of a wave's 64 rows is what it waits for) or as many as fit, at least 1.45x
+// the estimate.  Every workgroup fills, and merges, a table of its own, which
+// few rows don't pay for.  Measured, us a call, LDS / device-wide table, one
+// int64 sum: by value 1,000 slots 20K rows 110 / 103, 60K 118 / 120; 3,000 slots
+// 60K 142 / 120, 150K 130 / 146; 5,000 slots 150K 167 / 141, 250K 141 / 160
+// (partitioned from 200K); 9,000 slots 250K 208 / 158, 1.1M 172 / 172; by probe
+// 9,000 slots (3,000 groups) 150K 160 / 142, 600K 167 / 163.  Up to 512 slots
+// the two tie from the smallest calls on.  A key on 1/32 of the rows queues up on
+// its address in the device-wide table: 20K rows, Zipf(1.1) over 1,000 keys 109 /
+// 139.  In a fixed arena the tables are merged
+// straight into the device-wide one: 3,000 slots by value 150K 156 / 143, 1M
+// 168 / 262; 9,000 by probe 1M 251 / 241, 4M 300 / 429.
+int32_t groupby_call::lds_slots(bool& direct)
+{
+  direct = false;
+  if (P().key_mode != KM_INLINE || any_arg_ || nf_ > 64) return 0;
+  bool const queues = est_ <= 1024.0 && double(max_mult_) * 32.0 >= sampled_ && sampled_ > 0.0;
+  auto pays = [&](int32_t slots) {
+    return slots <= 512 || queues || double(N) >= 32768.0 + double(slots) * double(slots) / (mem_ ? 60.0 : 125.0);
+  };
+  int32_t const by_value = direct_slots();
+  if (by_value > 0 && pays(by_value)) {
+    direct = true;
+    return by_value;
+  }
+  int32_t const most = lds_most_slots();
+  if (est_ > double(LDS_PREAGG_MAX_GROUPS) || std::max(256.0, 1.45 * est_ + 64.0) > double(most)) return 0;
+  int32_t const probed = std::min<int32_t>(most, std::max<int32_t>(256, (int32_t(3.0 * est_) + 63) & ~63));
+  return pays(probed) ? probed : 0;
+}
+
+// Whether the call takes the LDS partial tables for all of its groups.
 bool groupby_call::few_groups()
 {
-  if (P().key_mode != KM_INLINE || any_arg_ || nf_ > 64) return false;
-  double const most = double(lds_most_slots());
-  return direct_slots() > 0 ||
-         (est_ <= double(LDS_PREAGG_MAX_GROUPS) && std::max(256.0, 1.45 * est_ + 64.0) <= most);
+  bool direct;
+  return lds_slots(direct) > 0;
 }
 
 // Slots of LDS tables indexed by an integer key's value: the sampled range,
@@ -1895,20 +1926,16 @@ int64_t groupby_call::aggregate_global()
   // workgroup-local tables for few groups, or for hot keys among many
   // groups (rows of keys that find no room go to the device-wide table)
   if (p.key_mode == KM_INLINE && !any_arg_ && forced != MIG_STRATEGY_PARTITIONED) {
-    // A third of the slots filled (the longest probe of a wave's 64 rows is
-    // what it waits for), or as many as fit.  Integer keys of a range that fits
-    // (ids, dictionary codes): a slot per key of the sampled range, found
-    // without probing.  Hot keys among many groups: as many slots as fit.
-    int32_t const most = lds_most_slots();
-    bool const few     = few_groups();
-    bool const hot     = !few && heavy_hitters() && most >= 1024;
-    int32_t S_l        = most;
-    if (few) S_l = std::min<int32_t>(most, std::max<int32_t>(256, (int32_t(3.0 * est_) + 63) & ~63));
-    int32_t const direct = direct_slots();
-    p.lds_direct         = direct > 0;
-    p.lds_key_min        = key_min_;
-    if (direct > 0) S_l = direct;
-    p.lds_hot = hot;
+    // Few groups: lds_slots.  Hot keys among many groups: as many slots as fit.
+    bool direct             = false;
+    int32_t const few_slots = lds_slots(direct);
+    int32_t const most      = lds_most_slots();
+    bool const few          = few_slots > 0;
+    bool const hot          = !few && heavy_hitters() && most >= 1024;
+    int32_t const S_l       = few ? few_slots : most;
+    p.lds_direct            = direct;
+    p.lds_key_min           = key_min_;
+    p.lds_hot               = hot;
     if (few || hot) lds_layout(S_l);
     if (p.lds_bytes > 0) {
       // one workgroup per CU (16 waves): more would only add tables to merge

@@ -184,3 +184,20 @@ def test_variance_when_the_hot_key_comes_last():
         _lib.set_phase_timing(False)
     assert st["lds_preagg"] == 1.0 and st["groups"] > 2.6 * st["est_groups"], st
     assert st["t_second_pass_ms"] < 4.0, st
+
+
+@pytest.mark.parametrize("n,card,spread,lds", [
+    (4_097, 170, 2**40, 1), (4_097, 1_500, 1, 0), (4_096, 20, 1, 0),   # up to 512 slots from the smallest estimated call on
+    (41_000, 1_024, 1, 0), (41_500, 1_024, 1, 1),                      # 1,024 slots by value
+    (90_000, 3_000, 2**40, 0), (900_000, 3_000, 2**40, 1),             # 9,000 by probe
+    (20_000, 10, 1_000, 1),                                            # a wide range of few keys: by probe
+])
+@pytest.mark.parametrize("kinds", [["SUM", "MIN"], ["MEAN", "VARIANCE"]])
+def test_rows_that_pay_for_tables(n, card, spread, lds, kinds):
+    """Both sides of the line between LDS tables and the device-wide table."""
+    rng = np.random.default_rng(n + card)
+    k = np.concatenate([np.arange(card), rng.integers(0, card, n - card)])[rng.permutation(n)] * spread
+    v = host_col(rng.integers(-1000, 1000, n))
+    assert assert_parity([host_col(k)], [(v, [(AGG[a], 1) for a in kinds])]) == card
+    if kinds[0] == "SUM" or card < 3_000:  # the variance tables hold fewer groups
+        assert _stats()["lds_preagg"] == lds, _stats()
