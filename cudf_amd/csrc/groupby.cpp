@@ -659,14 +659,19 @@ class groupby_call {
   int64_t hot_groups_ = 0;
   uint32_t* hot_map_  = nullptr;
   bool split_         = false;  // the partitioned path takes the spilled rows
-  // A key on at least 1/512 of the sampled rows among at most 2M groups: one
-  // bin of the partitioned path would hold that key's rows (a straggler
-  // workgroup), while the device-wide table of that many groups stays in the
-  // last-level cache and workgroup-local tables absorb the hot key.
+  // A key on at least 1/512 of the sampled rows, and on 4,096 rows or more,
+  // among at most 2M groups: one bin of the partitioned path would hold that
+  // key's rows (a straggler workgroup: LDS atomics on one address take 3.6 ns a
+  // row), while the device-wide table of that many groups stays in the last-level
+  // cache and workgroup-local tables absorb the hot key.  Fewer rows than that are
+  // a bin like the others, or a few wave-combined updates: 300K rows, four
+  // accumulators, 20 keys of 0.25% among 20,000 344 us a call with tables for them,
+  // 179 partitioned; 60K rows, one key of 2% 247 / 158 in the device-wide table.
   bool heavy_hitters() const
   {
-    return sampled_ > 0.0 && double(max_mult_) * 512.0 >= sampled_ && max_mult_ >= 16 &&
-           est_ <= double(1 << 21);
+    if (sampled_ <= 0.0 || max_mult_ < 16 || est_ > double(1 << 21)) return false;
+    double const share = double(max_mult_) / sampled_;
+    return share * 512.0 >= 1.0 && (N >= (1 << 20) || share * double(N) >= 4096.0);
   }
   int n_str_keys_ = 0;
   std::vector<string_out> string_outs_;
@@ -1926,7 +1931,11 @@ int64_t groupby_call::aggregate_global()
   // workgroup-local tables for few groups, or for hot keys among many
   // groups (rows of keys that find no room go to the device-wide table)
   if (p.key_mode == KM_INLINE && !any_arg_ && forced != MIG_STRATEGY_PARTITIONED) {
-    // Few groups: lds_slots.  Hot keys among many groups: as many slots as fit.
+    // Few groups: lds_slots.  Hot keys among many groups: as many slots as fit,
+    // half of them filled (every cold key's probe passes the filled ones), merged
+    // straight (most of their keys are in one table only).  250K rows, one key of
+    // 2% among 25,000, four accumulators 204 us a call; 0.85 filled, stored and
+    // merged 337; 2,048 slots 239.
     bool direct             = false;
     int32_t const few_slots = lds_slots(direct);
     int32_t const most      = lds_most_slots();
@@ -1937,6 +1946,7 @@ int64_t groupby_call::aggregate_global()
     p.lds_key_min           = key_min_;
     p.lds_hot               = hot;
     if (few || hot) lds_layout(S_l);
+    if (hot) p.lds_fill = p.lds_slots / 2;
     if (p.lds_bytes > 0) {
       // one workgroup per CU (16 waves): more would only add tables to merge
       // enough rows per group and workgroup that its table pays off (hot keys:
@@ -1966,7 +1976,7 @@ int64_t groupby_call::aggregate_global()
     p.overflow    = d_flags;
     p.special     = reinterpret_cast<uint32_t*>(d_flags + 1);
     stats_[STAT_STATE_BYTES] = double(alloc_table(cap));
-    alloc_dump(lds_blocks);
+    alloc_dump(p.lds_hot ? 0 : lds_blocks);
     upload(0);
     launch_init_state(dP, p, stream_);
     T->mark(2);

@@ -201,3 +201,23 @@ def test_rows_that_pay_for_tables(n, card, spread, lds, kinds):
     assert assert_parity([host_col(k)], [(v, [(AGG[a], 1) for a in kinds])]) == card
     if kinds[0] == "SUM" or card < 3_000:  # the variance tables hold fewer groups
         assert _stats()["lds_preagg"] == lds, _stats()
+
+
+@pytest.mark.parametrize("n,card,keys,share,lds,strategy", [
+    (60_000, 6_000, 1, 0.02, 0, 1),      # 1,200 rows of one key: an ordinary call
+    (300_000, 20_000, 20, 0.05, 0, 2),   # 750 rows each
+    (300_000, 25_000, 1, 0.01, 0, 2),
+    (300_000, 25_000, 1, 0.02, 1, 1),    # 6,000 rows: hot, tables half filled
+    (150_000, 50_000, 3, 0.3, 1, 1),
+])
+def test_hot_keys_by_their_rows(n, card, keys, share, lds, strategy):
+    """A key is hot by its rows as well as by its share of them."""
+    rng = np.random.default_rng(n + card)
+    k = rng.integers(0, card, n)
+    hot = rng.random(n) < share
+    k[hot] = rng.integers(0, keys, int(hot.sum()))
+    key = host_col(k * 1_000_003, rng.random(n) >= 0.005)
+    f = host_col(rng.standard_normal(n) + 3, rng.random(n) >= 0.04)
+    i = host_col(rng.integers(0, 10_000, n).astype(np.int32))
+    assert_parity([key], [(f, C2_AGGS), (i, C2_AGGS)], 1)
+    assert (_stats()["lds_preagg"], _stats()["strategy"]) == (lds, strategy), _stats()
