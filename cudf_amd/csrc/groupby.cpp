@@ -181,7 +181,9 @@ struct scratch_cache {
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
-      // release cached blocks of this device and try once more
+      // release cached blocks of this device and try once more (the first
+      // failure is not the error of a later launch)
+      (void)hipGetLastError();
       release_all(dev);
       e = hipMalloc(&p, bytes);
     }
@@ -234,6 +236,15 @@ struct scratch {
     void* p = scratch_cache::get().take(dev, bytes);
     blocks.emplace_back(p, bytes);
     return static_cast<T*>(p);
+  }
+  // Returns the blocks taken since there were `count` of them (nothing uses them
+  // any more).
+  void give_back(size_t count)
+  {
+    while (blocks.size() > count) {
+      scratch_cache::get().give(dev, blocks.back().first, blocks.back().second);
+      blocks.pop_back();
+    }
   }
   // Arena position, and a return to it (the blocks above it are free once
   // the work that used them has finished); no-ops for cached blocks.
@@ -535,8 +546,13 @@ owned_column make_owned_fixed(device_allocator& A, int32_t type_id, int64_t n, b
   oc.col.data       = n > 0 ? A.allocate(oc.data_bytes) : nullptr;
   oc.col.data_bytes = int64_t(oc.data_bytes);
   if (with_mask) {
-    oc.mask_bytes    = std::max<size_t>(8, size_t((n + 63) / 64) * 8);  // whole 64-bit words
-    oc.col.null_mask = static_cast<uint32_t*>(A.allocate(oc.mask_bytes));
+    oc.mask_bytes = std::max<size_t>(8, size_t((n + 63) / 64) * 8);  // whole 64-bit words
+    try {
+      oc.col.null_mask = static_cast<uint32_t*>(A.allocate(oc.mask_bytes));
+    } catch (...) {
+      A.deallocate(oc.col.data, oc.data_bytes);
+      throw;
+    }
     if (n == 0) MIG_HIP_TRY(hipMemsetAsync(oc.col.null_mask, 0, oc.mask_bytes, A.stream));
   }
   return oc;
@@ -700,10 +716,12 @@ class groupby_call {
   void upload(int which);
   void estimate_groups();
   owned_column fixed_output(int32_t type_id, int64_t rows_cap, int64_t G, bool with_mask, bool zero_masks);
+  void string_column(std::vector<owned_column>& to, int64_t G, size_t mask_bytes);
   void alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks);
   void release_outputs();
   void gather_general_keys(uint32_t const* rep_rows, int64_t G);
   int64_t aggregate_sorted_runs();
+  int64_t attempt(int64_t (groupby_call::*path)());
   int64_t aggregate_partitioned();
   int64_t aggregate_hot_split();
   bool partitionable();
@@ -1026,6 +1044,22 @@ owned_column groupby_call::fixed_output(int32_t type_id, int64_t rows_cap, int64
   return oc;
 }
 
+// A string column of `G` rows in `to`, its characters still to come; no mask when
+// `mask_bytes` is 0.  (In its place before the buffers are allocated, so that a
+// failed allocation leaves the first ones owned.)
+void groupby_call::string_column(std::vector<owned_column>& to, int64_t G, size_t mask_bytes)
+{
+  to.emplace_back();
+  owned_column& oc       = to.back();
+  oc.col.type_id         = MIG_TYPE_STRING;
+  oc.col.size            = int32_t(G);
+  oc.col.offsets_type_id = MIG_TYPE_INT32;
+  oc.offsets_bytes       = sizeof(int32_t) * size_t(G + 1);
+  oc.col.offsets         = A().allocate(oc.offsets_bytes);
+  oc.mask_bytes          = mask_bytes;
+  if (mask_bytes > 0) oc.col.null_mask = static_cast<uint32_t*>(A().allocate(mask_bytes));
+}
+
 // Output columns: keys, then the results in request order (duplicates
 // computed again from the same accumulators, as extract_results copies them).
 // Fixed-width columns get room for `rows_cap` rows and report `G` rows (the
@@ -1042,17 +1076,7 @@ void groupby_call::alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks)
   for (int i = 0; i < num_keys_; i++) {
     bool const with_mask = keys_[i].null_mask != nullptr;
     if (storage_of(keys_[i].type_id) == ST_STRING) {
-      owned_column oc;
-      oc.col.type_id         = MIG_TYPE_STRING;
-      oc.col.size            = int32_t(G);
-      oc.col.offsets_type_id = MIG_TYPE_INT32;
-      oc.offsets_bytes       = sizeof(int32_t) * size_t(G + 1);
-      oc.col.offsets         = A().allocate(oc.offsets_bytes);
-      if (with_mask) {
-        oc.mask_bytes    = std::max<size_t>(4, size_t((G + 31) / 32) * 4);
-        oc.col.null_mask = static_cast<uint32_t*>(A().allocate(oc.mask_bytes));
-      }
-      res_->keys.push_back(oc);
+      string_column(res_->keys, G, with_mask ? std::max<size_t>(4, size_t((G + 31) / 32) * 4) : 0);
       n_str_keys_++;
     } else {
       res_->keys.push_back(fixed_output(keys_[i].type_id, rows_cap, G, with_mask, zero_masks));
@@ -1064,7 +1088,8 @@ void groupby_call::alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks)
   int no = 0;
   for (int r = 0; r < num_requests_; r++) {
     value_plan const& vp = vals_[vcol_of_request_[r]];
-    std::vector<owned_column> cols;
+    res_->results.emplace_back();
+    std::vector<owned_column>& cols = res_->results.back();
     for (int a = 0; a < requests_[r].num_aggregations; a++) {
       int32_t const kind = requests_[r].aggregations[a].kind;
       int32_t const tt   = target_type_of(vp.view.type_id, kind);
@@ -1094,18 +1119,8 @@ void groupby_call::alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks)
             O.field   = kind == MIG_AGG_MIN ? vp.f_argmin : vp.f_argmax;
             O.data    = S->get<int32_t>(std::max<int64_t>(rows_cap, 1));
             O.mask    = nullptr;
-            owned_column oc;
-            oc.col.type_id         = MIG_TYPE_STRING;
-            oc.col.size            = int32_t(G);
-            oc.col.offsets_type_id = MIG_TYPE_INT32;
-            oc.offsets_bytes       = sizeof(int32_t) * size_t(G + 1);
-            oc.col.offsets         = A().allocate(oc.offsets_bytes);
-            if (vp.has_nulls) {
-              oc.mask_bytes    = std::max<size_t>(8, size_t((G + 63) / 64) * 8);
-              oc.col.null_mask = static_cast<uint32_t*>(A().allocate(oc.mask_bytes));
-            }
             string_outs_.push_back({r, int(cols.size()), vcol_of_request_[r], static_cast<int32_t*>(O.data)});
-            cols.push_back(oc);
+            string_column(cols, G, vp.has_nulls ? std::max<size_t>(8, size_t((G + 63) / 64) * 8) : 0);
             continue;
           }
           O.field = kind == MIG_AGG_MIN ? vp.f_min : vp.f_max;
@@ -1140,16 +1155,8 @@ void groupby_call::alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks)
             O.kind = OK_ARG;
             O.data = S->get<int32_t>(std::max<int64_t>(rows_cap, 1));
             O.mask = nullptr;
-            owned_column oc;
-            oc.col.type_id         = MIG_TYPE_STRING;
-            oc.col.size            = int32_t(G);
-            oc.col.offsets_type_id = MIG_TYPE_INT32;
-            oc.offsets_bytes       = sizeof(int32_t) * size_t(G + 1);
-            oc.col.offsets         = A().allocate(oc.offsets_bytes);
-            oc.mask_bytes          = std::max<size_t>(8, size_t((G + 63) / 64) * 8);
-            oc.col.null_mask       = static_cast<uint32_t*>(A().allocate(oc.mask_bytes));
             string_outs_.push_back({r, int(cols.size()), vcol_of_request_[r], static_cast<int32_t*>(O.data)});
-            cols.push_back(oc);
+            string_column(cols, G, std::max<size_t>(8, size_t((G + 63) / 64) * 8));
             continue;
           }
           break;
@@ -1172,7 +1179,6 @@ void groupby_call::alloc_outputs(int64_t rows_cap, int64_t G, bool zero_masks)
       O.mask          = oc.col.null_mask;
       cols.push_back(oc);
     }
-    res_->results.push_back(std::move(cols));
   }
   p.num_outs = no;
 }
@@ -1835,7 +1841,6 @@ int64_t groupby_call::aggregate_hot_split()
   lds_layout(slots);
   if (p.lds_bytes == 0) return -1;
   size_t const n       = size_t(N);
-  gb_params const keep = p;  // the original columns
   uint64_t const cap   = next_pow2(uint64_t(2 * slots));
   int32_t* d_flags     = S->get<int32_t>(4);  // [0] overflow, [1..2] special occupancy, [3] spilled rows
   p.cap         = cap;
@@ -1872,7 +1877,6 @@ int64_t groupby_call::aggregate_hot_split()
   MIG_HIP_TRY(hipMemcpyAsync(h + 4, block_counts + nb, 4, hipMemcpyDeviceToHost, stream_));
   MIG_HIP_TRY(hipStreamSynchronize(stream_));
   int64_t const spilled = int64_t(h[3]), hot = int64_t(h[4]);
-  double const est = est_, pop = pop_;
   int64_t G = -1;
   if (h[0] == 0 && spilled > 0) {
     hot_groups_ = hot;
@@ -1905,8 +1909,30 @@ int64_t groupby_call::aggregate_hot_split()
     stats_[STAT_LDS_PREAGG] = 1.0;
     stats_[STAT_STRATEGY]   = MIG_STRATEGY_GLOBAL;
   }
-  if (G < 0) {  // back to the whole input
-    p           = keep;
+  return G;
+}
+
+// A path that may not apply (-1).  The paths that move the rows, or make room for
+// more groups than there are, need memory that the device-wide table does not:
+// when an allocation fails, the automatic choice takes that table instead.
+// Either way the next path finds the whole input, and the memory given back.
+int64_t groupby_call::attempt(int64_t (groupby_call::*path)())
+{
+  gb_params const keep = P();
+  double const est = est_, pop = pop_;
+  size_t const blocks = S->blocks.size();
+  int64_t G           = -1;
+  try {
+    G = (this->*path)();
+  } catch (mig_error const& e) {
+    if (e.status != MIG_ERROR_ALLOC || mem_ || g_strategy.load() != MIG_STRATEGY_AUTO) throw;
+    (void)hipGetLastError();  // the failed allocation's
+    MIG_HIP_TRY(hipStreamSynchronize(stream_));
+    release_outputs();
+    S->give_back(blocks);
+  }
+  if (G < 0) {
+    P()         = keep;
     hot_groups_ = 0;
     split_      = false;
     est_        = est;
@@ -2153,11 +2179,11 @@ std::unique_ptr<mig_groupby_result> groupby_call::run()
   }
   if (G < 0) {
     func_range range("groupby: hot keys apart");
-    G = aggregate_hot_split();
+    G = attempt(&groupby_call::aggregate_hot_split);
   }
   if (G < 0) {
     func_range range("groupby: partitioned");
-    G = aggregate_partitioned();
+    G = attempt(&groupby_call::aggregate_partitioned);
   }
   if (G < 0) {
     func_range range("groupby: device-wide table");

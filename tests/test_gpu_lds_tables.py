@@ -221,3 +221,36 @@ def test_hot_keys_by_their_rows(n, card, keys, share, lds, strategy):
     i = host_col(rng.integers(0, 10_000, n).astype(np.int32))
     assert_parity([key], [(f, C2_AGGS), (i, C2_AGGS)], 1)
     assert (_stats()["lds_preagg"], _stats()["strategy"]) == (lds, strategy), _stats()
+
+
+@pytest.mark.parametrize("kind,n,card", [("one", 300_001, 6_000), ("general", 400_003, 3_000), ("hot", 1_100_003, 20_000)])
+def test_memory_for_the_groups_only(kind, n, card, monkeypatch):
+    """A memory resource with room for the groups found but not for what the
+    partitioned path may find: the call takes the device-wide table, and every
+    buffer of the attempt is given back."""
+    from cudf_amd import groupby
+    made = []
+
+    class Limited(groupby.TorchMemoryResource):
+        def __init__(self):
+            super().__init__()
+            self.refused = 0
+            made.append(self)
+
+        def _allocate(self, ctx, nbytes, stream):
+            if nbytes > 12 * card + 64:
+                self.refused += 1
+                return None
+            return super()._allocate(ctx, nbytes, stream)
+
+    monkeypatch.setattr(groupby, "TorchMemoryResource", Limited)
+    rng = np.random.default_rng(card)
+    k, x = _spread_over_mean(rng, n, card, kind)
+    key = host_col(k, rng.random(n) >= 0.01)
+    keys = [key] + ([host_col((k % 5).astype(np.int32))] if kind == "general" else [])
+    v = host_col(x, rng.random(n) >= 0.05)
+    i = host_col(rng.integers(-100, 100, n).astype(np.int32))
+    assert_parity(keys, [(v, [(AGG["SUM"], 1), (AGG["MAX"], 1), (AGG["VARIANCE"], 1)]),
+                         (i, [(AGG["SUM"], 1), (AGG["MIN"], 1), (AGG["COUNT_ALL"], 1)])], 1)
+    assert _stats()["strategy"] == 1
+    assert made[0].refused > 0 and not made[0].live
