@@ -757,7 +757,7 @@ def main():
                      "frac": achieved / HBM_PEAK, "traffic": traffic, "traffic_source": traffic_src,
                      "algorithmic_bytes": bytes_alg, "kernel_design_bytes": kernels[dom][1],
                      "avg_ms": t_dom * 1e3},
-        "pipeline": {"strategy": {1: "global", 2: "partitioned"}.get(int(st["strategy"]), "?"),
+        "pipeline": {"strategy": {1: "global", 2: "partitioned", 5: "hot keys apart"}.get(int(st["strategy"]), "?"),
                      "bytes_alg": in_b + out_b, "bytes_per_row": (in_b + out_b) / args.rows,
                      "achieved_GBps": (in_b + out_b) / (ms_per_step * 1e-3) / 1e9,
                      "frac": (in_b + out_b) / (ms_per_step * 1e-3) / HBM_PEAK,

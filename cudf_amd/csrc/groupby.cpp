@@ -1905,9 +1905,11 @@ int64_t groupby_call::aggregate_hot_split()
     split_    = true;
     G         = aggregate_partitioned();
   }
-  if (G >= 0) {  // reported as before: hot keys take the device-wide table with LDS tables in front
-    stats_[STAT_LDS_PREAGG] = 1.0;
-    stats_[STAT_STRATEGY]   = MIG_STRATEGY_GLOBAL;
+  if (G >= 0) {
+    stats_[STAT_LDS_PREAGG]   = 1.0;
+    stats_[STAT_STRATEGY]     = 5;  // hot keys apart
+    stats_[STAT_HOT_GROUPS]   = double(hot);
+    stats_[STAT_SPILLED_ROWS] = double(spilled);
   }
   return G;
 }

@@ -40,9 +40,9 @@ namespace mig {
 
 // Statistics of the last call on this thread (exposed by mig_last_stats).
 enum stat_index : int {
-  STAT_STRATEGY = 0,   // 0 = global table, 1 = LDS pre-aggregation
+  STAT_STRATEGY = 0,   // 1 table, 2 partitioned, 3 runs, 4 sort-based, 5 hot keys apart
   STAT_KEY_MODE,       // key_mode
-  STAT_CAPACITY,       // table slots
+  STAT_CAPACITY,       // table slots (partitioned: bins)
   STAT_EST_GROUPS,     // estimated groups
   STAT_GROUPS,         // actual groups
   STAT_RETRIES,        // table rebuilds after overflow
@@ -57,9 +57,11 @@ enum stat_index : int {
   STAT_T_RPA_SCATTER1,
   STAT_T_RPA_SCATTER2,
   STAT_T_RPA_AGGREGATE,
-  STAT_LDS_PREAGG,       // 1 when the global path pre-aggregated in LDS
+  STAT_LDS_PREAGG,       // 1 when LDS tables aggregated rows outside the partitioned path
   STAT_RPA_SPECULATIVE,  // 1 when the partitioned path's bins were sized without a histogram
-  STAT_VERIFIED_PAIRS,   // general keys, hashed form: rows compared with their group's representative
+  STAT_VERIFIED_PAIRS,   // general keys, hashed form: rows compared with their group's key
+  STAT_HOT_GROUPS,       // hot keys apart: groups of the LDS tables
+  STAT_SPILLED_ROWS,     // and rows of the partitioned path
   STAT_COUNT
 };
 double* thread_stats();

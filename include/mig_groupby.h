@@ -380,10 +380,16 @@ void mig_result_free(mig_groupby_result* r);
 /* Statistics of the last mig_groupby_aggregate call on this thread, for
  * benchmarks and the autotuner (strategy chosen, table capacity, time per
  * phase).  Writes at most `n` doubles; returns the number available.
- * Index: 0 strategy, 1 key mode, 2 table slots, 3 estimated groups,
- * 4 groups, 5 table rebuilds, 6 state bytes, then phase times in ms
- * (7 estimate, 8 init, 9 accumulate, 10 second pass, 11 compact,
- * 12 outputs) when phase timing is on. */
+ * Index: 0 strategy (1 device-wide table, 2 partitioned, 3 runs of pre-sorted
+ * keys, 4 sort-based, 5 hot keys in workgroup-local tables and the other rows
+ * partitioned), 1 key mode, 2 table slots (2 and 5: bins; 3: groups),
+ * 3 estimated groups, 4 groups, 5 table rebuilds, 6 state bytes, then phase
+ * times in ms (7 estimate, 8 init, 9 accumulate, 10 second pass, 11 compact,
+ * 12 outputs, 13 to 16 the partitioned path's histogram, two scatters and
+ * aggregation) when phase timing is on; 17 whether workgroup-local tables took
+ * part, 18 whether the bins were sized without a histogram, 19 rows verified
+ * against their group's key; of strategy 5: 20 groups taken by the tables (hot
+ * keys, and the null key's), 21 rows partitioned. */
 int32_t mig_last_stats(double* values, int32_t n);
 
 /* Turns hipEvent timing of each phase of mig_groupby_aggregate on (1) or off
