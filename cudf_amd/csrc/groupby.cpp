@@ -968,6 +968,7 @@ void groupby_call::estimate_groups()
   if (N > 4096 && !keys_sorted_) {
     int64_t const ns = std::min<int64_t>(N, SAMPLE_ROWS);
     uint32_t const tslots = uint32_t(next_pow2(uint64_t(2 * ns)));
+    size_t const before = S->mark();
     auto* table    = S->get<uint64_t>(tslots);
     sample_table_  = table;
     sample_mask_   = tslots - 1;
@@ -987,6 +988,7 @@ void groupby_call::estimate_groups()
     MIG_HIP_TRY(hipMemcpyAsync(hr, d_ranges, sizeof(int64_t) * nranges + sizeof(uint32_t) * NSTATS,
                                hipMemcpyDeviceToHost, stream_));
     MIG_HIP_TRY(hipStreamSynchronize(stream_));
+    S->release_to(before);  // an arena has no other use for the sample (aggregate_hot_split)
     for (int64_t b = 0; ranged && b < nranges; b += 2) {
       key_min_ = std::min(key_min_, hr[b]);
       key_max_ = std::max(key_max_, hr[b + 1]);

@@ -170,3 +170,49 @@ def test_no_alloc_rejects_small_outputs_and_oversized_tables():
     # and the entry point still works afterwards
     _compare(20_000, 500, 4)
     del keep, bufs
+
+
+def test_no_alloc_tables_have_the_whole_scratch():
+    """A call whose tables take 127.3 of the 128 MiB: what the estimate read its
+    sample into (1 MiB here) is theirs too."""
+    import torch
+    from cudf_amd import _lib
+    n, card = 65_536, 60_000  # 2^18 slots of 8 + 62 x 8 + 4 bytes
+    rng = np.random.default_rng(8)
+    k = rng.permutation(np.concatenate([np.arange(card), rng.integers(0, card, n - card)])).astype(np.int64) * 7
+    base = rng.integers(-10**9, 10**9, n)
+    cols = [base + c for c in range(31)] + [base.astype(np.int32)]
+    kinds = [[AGG["SUM"], AGG["MIN"]]] * 31 + [[AGG["MIN"]]]
+    dk, dvals = to_device(host_col(k)), [to_device(host_col(c)) for c in cols]
+    keys = (_lib.ColumnView * 1)(dk.view())
+    reqs, keep, bufs, outs = (_lib.AggregationRequest * 32)(), [], [], []
+
+    def out(width):
+        d, c = torch.empty(n * width, dtype=torch.uint8, device="cuda"), _lib.OutColumn()
+        c.data, c.data_bytes = d.data_ptr(), n * width
+        bufs.append(d)
+        return c
+
+    out_k = (_lib.OutColumn * 1)(out(8))
+    for r, (v, ks) in enumerate(zip(dvals, kinds)):
+        aggs = (_lib.Aggregation * len(ks))(*[_lib.Aggregation(a, 1) for a in ks])
+        keep.append(aggs)
+        reqs[r].values, reqs[r].aggregations, reqs[r].num_aggregations = v.view(), aggs, len(ks)
+        outs += [out(4 if r == 31 else 8) for _ in ks]
+    out_r = (_lib.OutColumn * len(outs))(*outs)
+    g = ctypes.c_int32(-1)
+    torch.cuda.synchronize()
+    _lib.check(_lib.lib().mig_groupby_aggregate_into(keys, 1, 0, reqs, 32, out_k, out_r, ctypes.byref(g), None))
+    assert g.value == card
+    ids = bufs[0].cpu().numpy().view(np.int64)[:card]
+    order = np.argsort(ids)
+    assert np.array_equal(ids[order], np.arange(card) * 7)
+    by_key = np.argsort(k, kind="stable")
+    first = np.searchsorted(k[by_key], np.arange(card) * 7)
+    for c in (0, 30):
+        x = cols[c][by_key]
+        assert np.array_equal(bufs[1 + 2 * c].cpu().numpy().view(np.int64)[:card][order], np.add.reduceat(x, first))
+        assert np.array_equal(bufs[2 + 2 * c].cpu().numpy().view(np.int64)[:card][order], np.minimum.reduceat(x, first))
+    assert np.array_equal(bufs[63].cpu().numpy().view(np.int32)[:card][order],
+                          np.minimum.reduceat(cols[31][by_key], first))
+    del keep
