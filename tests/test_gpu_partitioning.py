@@ -346,3 +346,29 @@ def test_partition_tile_edges(rows, nparts):
     cols = [host_col(rng.integers(0, 1 << 40, rows)), host_col(rng.integers(-100, 100, rows).astype(np.int8)),
             host_col(rng.integers(0, 9, rows).astype(np.int16)), host_col(rng.normal(size=rows).astype(np.float32))]
     _check_hash_partition(cols, [0], nparts)
+
+
+@pytest.mark.parametrize("nparts", [7, 3000])
+@pytest.mark.parametrize("rows", [1, 513, 100_003, 600_001, 1_200_003, 2_200_001])
+def test_partition_sixteen_byte_elements_and_row_maps(rows, nparts):
+    """Elements of 16 bytes (moved as two halves) first, between other widths
+    and last; with more than 2,048 partitions the second pass reads its rows
+    through a map.  Both at every tile size: exact against the oracle's order."""
+    import torch
+    from cudf_amd import Column, Table, TypeId
+    from cudf_amd.partitioning import hash_partition
+    rng = np.random.default_rng(rows + nparts)
+    key = host_col(rng.integers(0, 1 << 40, rows))
+    wide = [rng.integers(0, 256, (rows, 16), dtype=np.uint8) for _ in range(3)]
+    byte, four, eight = (host_col(rng.integers(-100, 100, rows).astype(t)) for t in (np.int8, np.int32, np.float64))
+    dec = [Column(TypeId.DECIMAL128, rows, torch.from_numpy(w.reshape(-1)).cuda()) for w in wide]
+    table = Table([dec[0], to_device(key), to_device(byte), dec[1], to_device(four), to_device(eight), dec[2]])
+    order, offs = po.hash_partition([key, byte, four, eight], [0], nparts)
+    out, got_offs = hash_partition(table, [1], nparts)
+    assert got_offs == offs
+    cols = out.columns()
+    for i, c in ((1, key), (2, byte), (4, four), (5, eight)):
+        _assert_col_equal(cols[i], po.gather(c, order), f"column {i}")
+    for i, w in ((0, wide[0]), (3, wide[1]), (6, wide[2])):
+        assert cols[i].type_id == TypeId.DECIMAL128
+        assert np.array_equal(cols[i].data[:16 * rows].cpu().numpy().reshape(rows, 16), w[order]), f"column {i}"
