@@ -1345,10 +1345,13 @@ bool groupby_call::partitionable()
 // 120K rows 148 / 152, 240K 160 / 157, 1M 213 / 183, 16M 1,022 / 567; four
 // accumulators 60K 158 / 160, 240K 205 / 170, 4M 861 / 262, 16M 2,962 / 613
 // (5,000 to N / 3 groups alike).  Few groups take the LDS tables instead.
-// General keys (hashing and verifying rows costs more): five accumulators
-// 100K 280 / 310, 300K 355 / 325, 6M 1,847 / 995; one accumulator no gain
-// (300K 282 / 291, 6M 846 / 895) but with few groups (600: 300K 376 / 292, 6M
-// 2,069 / 994).  A key on many rows would make a straggler of its bin.
+// General keys (hashing and verifying rows costs more; two integers, 5,000 to N / 3
+// groups): one accumulator no gain (700K 195 / 242, 6M 496 / 698), two from 6M on
+// (2M 337 / 342, 6M 714 / 714), three 300K 206 / 231, 700K 258 / 252, 2M 419 / 348,
+// four 300K 224 / 234, 700K 288 / 262, five 300K 355 / 325, 6M 1,847 / 995.  Few
+// groups queue up in the table: 600 groups, one accumulator 300K 241 / 225, 6M
+// 910 / 754.  An integer and a string: three accumulators 300K 276 / 281, 700K
+// 337 / 319.  A key on many rows would make a straggler of its bin.
 bool groupby_call::partitioning_pays()
 {
   gb_params const& p  = P();
@@ -1356,7 +1359,8 @@ bool groupby_call::partitioning_pays()
   if (p.key_mode == KM_INLINE) return N >= 200'000 && !few_groups() && !heavy_hitters();
   if (high_cardinality()) return !heavy_hitters();
   bool const straggler = sampled_ > 0.0 && double(max_mult_) * 64.0 >= sampled_;
-  return N >= 300'000 && (atomics >= 3 || est_ <= 1024.0) && !straggler;
+  bool const many      = atomics >= 3 && double(N) * double(atomics - 1) >= 1.2e6;
+  return N >= 300'000 && (many || est_ <= 1024.0) && !straggler;
 }
 
 // Sizes at which every kind of key is partitioned (unless some key is hot).

@@ -255,3 +255,16 @@ def test_memory_for_the_groups_only(kind, n, card, monkeypatch):
                          (i, [(AGG["SUM"], 1), (AGG["MIN"], 1), (AGG["COUNT_ALL"], 1)])], 1)
     assert _stats()["strategy"] == 1
     assert made[0].refused > 0 and not made[0].live
+
+
+@pytest.mark.parametrize("n,card,kinds,strategy", [
+    (590_000, 9_000, ["SUM", "MIN", "MAX"], 1), (610_000, 9_000, ["SUM", "MIN", "MAX"], 2),
+    (390_000, 9_000, ["SUM", "MIN", "MAX", "COUNT_ALL"], 1), (410_000, 9_000, ["SUM", "MIN", "MAX", "COUNT_ALL"], 2),
+    (700_000, 9_000, ["SUM", "MAX"], 1), (310_000, 900, ["SUM"], 2),
+])
+def test_path_of_general_keys_by_accumulators(n, card, kinds, strategy):
+    rng = np.random.default_rng(n)
+    k = rng.integers(0, card, n)
+    v = host_col(rng.integers(-1000, 1000, n))
+    assert_parity([host_col((k % 89).astype(np.int16)), host_col(k)], [(v, [(AGG[a], 1) for a in kinds])])
+    assert _stats()["strategy"] == strategy, _stats()
