@@ -1961,15 +1961,17 @@ int64_t groupby_call::aggregate_global()
   int const forced   = g_strategy.load();
   uint64_t const max_cap = next_pow2(uint64_t(2 * N + 2));
   int64_t lds_blocks = 0;
+  bool merge_straight = false;
   p.lds_bytes        = 0;
   // workgroup-local tables for few groups, or for hot keys among many
   // groups (rows of keys that find no room go to the device-wide table)
   if (p.key_mode == KM_INLINE && !any_arg_ && forced != MIG_STRATEGY_PARTITIONED) {
     // Few groups: lds_slots.  Hot keys among many groups: as many slots as fit,
     // half of them filled (every cold key's probe passes the filled ones), merged
-    // straight (most of their keys are in one table only).  250K rows, one key of
+    // straight when most of their keys are in one table only.  250K rows, one key of
     // 2% among 25,000, four accumulators 204 us a call; 0.85 filled, stored and
-    // merged 337; 2,048 slots 239.
+    // merged 337; 2,048 slots 239.  1M rows, one key of 60% among 3,000, two columns:
+    // merged straight 372, stored and merged 293.
     bool direct             = false;
     int32_t const few_slots = lds_slots(direct);
     int32_t const most      = lds_most_slots();
@@ -1981,6 +1983,7 @@ int64_t groupby_call::aggregate_global()
     p.lds_hot               = hot;
     if (few || hot) lds_layout(S_l);
     if (hot) p.lds_fill = p.lds_slots / 2;
+    merge_straight = hot && est_ > 2.0 * double(p.lds_slots);
     if (p.lds_bytes > 0) {
       // one workgroup per CU (16 waves): more would only add tables to merge
       // enough rows per group and workgroup that its table pays off (hot keys:
@@ -2010,7 +2013,7 @@ int64_t groupby_call::aggregate_global()
     p.overflow    = d_flags;
     p.special     = reinterpret_cast<uint32_t*>(d_flags + 1);
     stats_[STAT_STATE_BYTES] = double(alloc_table(cap));
-    alloc_dump(p.lds_hot ? 0 : lds_blocks);
+    alloc_dump(merge_straight ? 0 : lds_blocks);
     upload(0);
     launch_init_state(dP, p, stream_);
     T->mark(2);
