@@ -101,7 +101,9 @@ class BatchedGroupBy:
     def result(self, i: int) -> Tuple[Table, List[Table]]:
         """Instance ``i``'s unique keys and per-request results, copied out of
         the plan's buffers on torch's current stream (valid after
-        ``synchronize``, on the stream the plan ran on or one ordered after it)."""
+        ``synchronize``, on the stream the plan ran on or one ordered after it).
+        The columns are slices of one tensor: a column that is kept keeps the
+        instance's others allocated too, unless it is cloned."""
         L = _lib.lib()
         n = 1 + sum(len(al) for al in self._aggs)
         cols = (_lib.OutColumn * n)()

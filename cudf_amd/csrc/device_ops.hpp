@@ -123,10 +123,10 @@ __device__ __forceinline__ uint64_t load_tail(gmem<uint8_t const>* p, int n)
   return a | (b << (8 * (n >> 1))) | (c << (8 * (n - 1)));
 }
 
-// MurmurHash3_x86_32 of `len` bytes under two seeds: mm_hash_bytes' hash, read
-// 8 bytes at a time whatever the alignment.  A wave's strings lie on lines of
-// their own, so the number of load instructions is what counts: hashing and
-// verifying 10M (integer, string) keys byte by byte took 0.75 ms more.
+// MurmurHash3_x86_32 of `len` bytes under two seeds, read 8 bytes at a time
+// whatever the alignment.  A wave's strings lie on lines of their own, so the
+// number of load instructions is what counts: hashing and verifying 10M
+// (integer, string) keys byte by byte took 0.75 ms more.
 __device__ __forceinline__ void str_hash2(gmem<uint8_t const>* p, int64_t len, uint32_t s1, uint32_t s2, uint32_t& o1,
                                           uint32_t& o2)
 {

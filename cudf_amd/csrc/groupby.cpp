@@ -47,9 +47,10 @@ constexpr int32_t RPA_LDS_BUDGET     = 80 * 1024;  // two aggregating workgroups
 constexpr int RPA_MAX_LOG_BINS       = 16;  // 256 x 256 through the two scatter passes
 constexpr int RPA_MAX_LOG_FANOUT     = 8;
 constexpr int32_t RPA_STAGE_BUDGET   = 56 * 1024;  // LDS staging of a scatter tile (3 workgroups per CU)
-// Global path, low cardinality: LDS partial tables, used when the estimate is
-// at most LDS_PREAGG_MAX_GROUPS groups and their table fits; one workgroup per CU, whose 160 KB
-// also hold its 8 KB of rows that found no room.
+// Global path, low cardinality: LDS partial tables (lds_slots); probed ones for
+// an estimate of at most LDS_PREAGG_MAX_GROUPS groups, those indexed by value up
+// to the slots that fit.  One workgroup per CU, whose 160 KB also hold its 8 KB of
+// rows that found no room.
 constexpr int32_t LDS_PREAGG_MAX_GROUPS = 4096;
 constexpr int32_t LDS_PREAGG_BUDGET     = 144 * 1024;
 // Up to this many workgroups merge their tables straight into the device-wide

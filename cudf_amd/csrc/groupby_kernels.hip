@@ -688,7 +688,9 @@ __device__ __forceinline__ void lds_insert_rows(uint64_t* tkeys, uint32_t* fill,
   uint32_t pos[N];
 #pragma unroll
   for (int u = 0; u < N; u++) pos[u] = lds_first_slot(h[u], S);
-  // S + N rounds pass every slot; the table is never full, so no row needs them
+  // S rounds pass every slot.  `limit` is soft (threads that read the count
+  // together all insert), so a small table can fill up: a key that is in it is
+  // found, any other row leaves after the S rounds with -1.
   for (int p = 0; p < S && pending != 0; p++) {
     uint64_t cur[N];
 #pragma unroll

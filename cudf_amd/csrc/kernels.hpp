@@ -169,7 +169,7 @@ struct gb_params {
   void* out_keys[MAX_KEYS];       // fixed-width key outputs (or string offsets)
   uint32_t* out_key_mask[MAX_KEYS];
   // low-cardinality pre-aggregation (inline keys): each workgroup keeps an
-  // LDS table of lds_slots keys (at most lds_fill; lds_slots + LDS_EXTRA_SLOTS
+  // LDS table of lds_slots keys (about lds_fill at most; lds_slots + LDS_EXTRA_SLOTS
   // words) with partials at
   // fields[f].lds_off (lds_slots + LDS_EXTRA_SLOTS elements of the field's
   // width; slots lds_slots and lds_slots + 1 hold the EMPTY_KEY and null-key
@@ -289,7 +289,7 @@ struct rpa_params {
   uint32_t* rep_rows;
   uint32_t* rec_slot;                // [input rows]
   int64_t rec_count;                 // input rows (the verification's range)
-  unsigned long long* verified;      // rows compared with a representative
+  unsigned long long* verified;      // rows compared with their group's key
   int32_t* verify_failed;
   // Pass-A plan of the aggregate kernel, read into registers once per
   // workgroup: the accumulators of value column plan_col[i] are the fields
@@ -498,7 +498,7 @@ void launch_rpa_scatter2(gb_params const* dP, rpa_params const* dR, rpa_params c
 // 1 general keys compared row by row, 2 general keys in hashed form
 void launch_rpa_aggregate(gb_params const* dP, rpa_params const* dR, rpa_params const& hR, int key_form,
                           int64_t bin_begin, int64_t bin_end, hipStream_t s);
-// exact key comparison of the (row, representative) pairs of the hashed form
+// exact key comparison of the hashed form's rows with their groups' result keys
 struct key_columns {  // the result's key columns
   dcol col[MAX_KEYS];
 };

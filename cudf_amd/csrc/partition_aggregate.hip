@@ -613,7 +613,7 @@ __global__ void __launch_bounds__(RPA_AGG_BLOCK) __attribute__((amdgpu_waves_per
     bool const in_range = live && pos < cap;
     bool const kvalid   = slot != S;
     if (live && !in_range) astore(R.overflow, 1);
-    if (KM == KF_HASHED) {  // keys are gathered from the representative rows afterwards
+    if (KM == KF_HASHED) {  // keys are gathered from the representative input rows afterwards
       if (in_range) {
         auto const rep     = gp(R.rep_rows) + rbase + slot;
         gp(R.out_rep)[pos] = __hip_atomic_load(rep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -580,7 +580,7 @@ hp_ranges hp_plan(int64_t n, int bits, int num_cus)
   while (r.rpt > 1 && n < int64_t(HP_TILE_BLOCK) * r.rpt * 2 * num_cus) r.rpt /= 2;
   int64_t const tile  = int64_t(HP_TILE_BLOCK) * r.rpt;
   int64_t const tiles = (n + tile - 1) / tile;
-  // ranges: four rounds of the three workgroups a CU holds, and a digit-major
+  // ranges: six rounds of the two workgroups a CU holds, and a digit-major
   // histogram of at most 2^22 counters
   int64_t const most = std::max<int64_t>(64, std::min<int64_t>(int64_t(num_cus) * 12, (int64_t(1) << 22) >> bits));
   r.per = (tiles + most - 1) / most * tile;
