@@ -653,6 +653,7 @@ class groupby_call {
   bool needs_sort_ = false;
   std::unique_ptr<mig_groupby_result> res_;
   std::unique_ptr<gb_params> P_ptr_;
+  std::unique_ptr<gb_params> kept_;  // as they were before the path being tried
   gb_params* Pp_ = nullptr;
   gb_params* dP = nullptr;
   uint8_t* pin = nullptr;
@@ -723,6 +724,10 @@ class groupby_call {
   void gather_general_keys(uint32_t const* rep_rows, int64_t G);
   int64_t aggregate_sorted_runs();
   int64_t attempt(int64_t (groupby_call::*path)());
+  void keep_params()
+  {
+    if (!kept_) kept_ = std::make_unique<gb_params>(P());
+  }
   int64_t aggregate_partitioned();
   int64_t aggregate_hot_split();
   bool partitionable();
@@ -1422,6 +1427,7 @@ int64_t groupby_call::aggregate_partitioned()
   else if (forced == MIG_STRATEGY_AUTO)  // and the estimate fits the largest partition
     use_rpa = rpa_ok && (split_ || partitioning_pays()) && est_ <= double(int64_t(1) << RPA_MAX_LOG_BINS) * max_fill;
   if (!use_rpa) return -1;
+  keep_params();
   int64_t const rows = p.num_rows;  // the input's, or those left after aggregate_hot_split
 
   int const num_cus = props().num_cus;
@@ -1843,6 +1849,7 @@ int64_t groupby_call::aggregate_hot_split()
   while (level < SAMPLE_HOT_LEVELS && hot_hashes_[level] > uint32_t(slots / 2)) level++;
   if (level == SAMPLE_HOT_LEVELS || hot_hashes_[level] == 0) return -1;
   uint32_t const at_least = uint32_t(SAMPLE_HOT_MIN) << level;
+  keep_params();
   p.lds_bytes  = 0;
   p.lds_direct = 0;
   lds_layout(slots);
@@ -1924,13 +1931,14 @@ int64_t groupby_call::aggregate_hot_split()
 // A path that may not apply (-1).  The paths that move the rows, or make room for
 // more groups than there are, need memory that the device-wide table does not:
 // when an allocation fails, the automatic choice takes that table instead.
-// Either way the next path finds the whole input, and the memory given back.
+// Either way the next path finds the whole input (a path calls keep_params once it
+// is sure to apply), and the memory given back.
 int64_t groupby_call::attempt(int64_t (groupby_call::*path)())
 {
-  gb_params const keep = P();
   double const est = est_, pop = pop_;
   size_t const blocks = S->blocks.size();
   int64_t G           = -1;
+  kept_.reset();
   try {
     G = (this->*path)();
   } catch (mig_error const& e) {
@@ -1940,8 +1948,8 @@ int64_t groupby_call::attempt(int64_t (groupby_call::*path)())
     release_outputs();
     S->give_back(blocks);
   }
-  if (G < 0) {
-    P()         = keep;
+  if (G < 0 && kept_) {
+    P()         = *kept_;
     hot_groups_ = 0;
     split_      = false;
     est_        = est;
